@@ -173,6 +173,36 @@ def test_empty_and_degenerate_inputs():
     assert h["t"][0] == pytest.approx(0.5, rel=1e-6) and h["t"][2] == pytest.approx(0.5, rel=1e-6)
 
 
+@pytest.mark.parametrize("scale", [1e-3, 1.0, 1e4])
+@pytest.mark.parametrize("length", [1e-6, 1.0, 1e6])
+def test_trace_scaled_scenes_and_directions(scale, length):
+    """Scene sizes and direction lengths far from 1, with rays along one axis
+    and in a coordinate plane (the divisions of their set-up) and in any
+    direction (its multiply-adds), some with an upper end inside the scene."""
+    d = ngi.Scene.generate(ngi.GEN_BATCH_ROOM, 5, 1.0, 600).desc()
+    s = ngi.Scene.create(d["positions"] * scale, d["faces"], d["tri_prim"], d["primitives"], normals=d["normals"])
+    s.build(ngi.BVH_8)
+    rng = np.random.default_rng(9)
+    n = 6000
+    o = rng.uniform(0.02, 0.98, (n, 3)) * scale
+    w = rng.normal(size=(n, 3))
+    w[:1000] *= np.eye(3)[rng.integers(0, 3, 1000)]
+    w[1000:2000] *= 1.0 - np.eye(3)[rng.integers(0, 3, 1000)]
+    w /= np.linalg.norm(w, axis=1, keepdims=True)
+    rays = ngi.make_rays(o, w * length, tmin=1e-5 * scale / length)
+    rays["tmax"][::3] = (rng.uniform(0.05, 1.0, len(rays[::3])) * scale / length).astype(np.float32)
+    # Distances in units of the scene, so that the comparison's bar means the same at every scale.
+    g, ref = s.trace(rays), oracle.trace(s, rays, use_bvh=False)
+    gh, oh = g["tri"] != ngi.MISS, ref["tri"] != ngi.MISS
+    assert (gh != oh).sum() <= int(5e-4 * n)
+    both = gh & oh
+    tg, to = (x["t"][both].astype(np.float64) * length / scale for x in (g, ref))
+    assert (np.abs(tg - to) <= T_RTOL * np.maximum(1.0, to)).mean() >= 0.9995
+    assert both.mean() > 0.5
+    occluded = s.trace(rays, any_hit=True)["tri"] != ngi.MISS
+    assert (occluded != gh).sum() == 0
+
+
 def test_trace_full_sphere_field_against_oracle_bvh():
     """The benchmark's 1,833,314-triangle scene (displaced icosphere on a
     512^2 heightfield), 10^6 rays: half from random points of the scene's
