@@ -167,7 +167,7 @@ int device_prepare(HostScene& s) {
     v.num_tris = (uint32_t)nt;
     v.sensor_prim = s.sensor_prim;
     // Geometry in leaf order.
-    std::vector<float4> tris(3 * nt), shade(3 * nt);
+    std::vector<float4> tris(3 * nt + (nt ? 1 : 0)), shade(3 * nt);   // fetch_child reads a float4 past the last triangle
     for (size_t j = 0; j < nt; ++j) {
         const uint32_t t = s.bvh.leaf_to_tri[j];
         for (int k = 0; k < 3; ++k) {

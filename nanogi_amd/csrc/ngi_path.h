@@ -212,7 +212,7 @@ __device__ __forceinline__ void shq_drain(const RenderArgs& a, const ShadowQueue
                 tmax = sr.tmax;
                 cur = 0;
                 sp = 0;
-                mask = sc.num_tris ? visit8<COUNT>(sc, r, 0, NGI_EPS_F, tmax, tc) : 0u;
+                mask = sc.num_tris ? NGI_TRAV8_FRESH : 0u;
                 busy = true;
                 cnt[CNT_SHADOW_RAYS]++;
             }
@@ -233,19 +233,16 @@ __device__ __forceinline__ void shq_drain(const RenderArgs& a, const ShadowQueue
             }
         }
         if (busy) {
-            const uint32_t i = __builtin_ctz(mask);
+            const int32_t ref = mask == NGI_TRAV8_FRESH ? 0 : next_child(sc, r, cur, mask);
             mask &= mask - 1u;
-            const uint32_t slot = i ^ r.octant;
-            const int32_t ref = reinterpret_cast<const int32_t*>(sc.nodes + 8 * (size_t)cur + 4)[slot];
-            if (ref >= 0) {
+            const Fetch f = fetch_child(sc, ref);
+            if (ref < 0) {
+                TraceHit h;
+                if (leaf_test<true, COUNT>(sc, r, ref, f, NGI_EPS_F, tmax, h, tc)) busy = false;
+            } else {
                 if (mask) stk[(sp++) * stride] = (cur << 8) | mask;
                 cur = (uint32_t)ref;
-                mask = visit8<COUNT>(sc, r, cur, NGI_EPS_F, tmax, tc);
-            } else {
-                TraceHit h;
-                bool occluded = false;
-                leaf_test<true, COUNT>(sc, r, ref, NGI_EPS_F, tmax, h, tc, occluded);
-                if (occluded) busy = false;
+                mask = visit8<COUNT>(f, r, NGI_EPS_F, tmax, tc);
             }
         }
     }

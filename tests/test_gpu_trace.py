@@ -17,6 +17,7 @@ import pytest
 
 import nanogi_amd as ngi
 import oracle
+from tests.scenes import SceneBuilder
 
 pytestmark = pytest.mark.gpu
 
@@ -171,6 +172,26 @@ def test_empty_and_degenerate_inputs():
     assert h["tri"][0] != ngi.MISS and h["tri"][1] == ngi.MISS and h["tri"][2] != ngi.MISS
     # Axis-aligned rays (zero direction components) hit the walls at exact distances.
     assert h["t"][0] == pytest.approx(0.5, rel=1e-6) and h["t"][2] == pytest.approx(0.5, rel=1e-6)
+
+
+@pytest.mark.parametrize("width", [ngi.BVH_2, ngi.BVH_8])
+@pytest.mark.parametrize("tris,leaf", [(1, 4), (2, 1), (2, 4), (3, 3), (5, 16), (16, 16), (17, 16), (33, 1)])
+def test_trace_leaf_sizes(width, tris, leaf):
+    """Leaves of one triangle (the last of the array among them), of two and
+    of more, against the brute-force oracle."""
+    rng = np.random.default_rng(100 * tris + leaf)
+    B = SceneBuilder()
+    p = B.prim(type=ngi.PRIM_D, D_R=(0.5, 0.5, 0.5))
+    for _ in range(tris):
+        c = rng.uniform(0.0, 1.0, 3)
+        B.tri(p, *(c + rng.uniform(-0.3, 0.3, (3, 3))))
+    B.camera((0.5, 0.5, 3.0), (0.5, 0.5, 0.0))
+    s = B.scene()
+    s.build(width, max_leaf_size=leaf)
+    rays = _random_rays([-0.5] * 3, [1.5] * 3, 4000, tris)
+    g, _ = _compare(s, rays, use_bvh=False)
+    occluded = s.trace(rays, any_hit=True)["tri"] != ngi.MISS
+    assert np.array_equal(occluded, g["tri"] != ngi.MISS)
 
 
 @pytest.mark.parametrize("scale", [1e-3, 1.0, 1e4])
