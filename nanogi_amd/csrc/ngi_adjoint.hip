@@ -420,6 +420,11 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_resume_k
                 active = false;
             }
         }
+        // Read by the steps above only, and written anew before the next ones
+        // (as forget_vertex).
+        s.gn = s.n = wi = f3(0.0f);
+        s.degenerate = false;
+        type = prim = 0;
         if (__ballot(active) == 0) {
             if (exhausted) break;
             continue;

@@ -268,6 +268,7 @@ __global__ void __launch_bounds__(BLOCK, NGI_BATCH_WAVES) batch_resume_kernel(Ba
                 ended_now = true;
             }
         }
+        forget_vertex(ps);
         ended += (unsigned long long)__popcll(__ballot(ended_now));
         const bool any = __ballot(active) != 0;
         // All queued rays are traced before the wave leaves the scene.

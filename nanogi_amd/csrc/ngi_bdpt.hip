@@ -734,6 +734,10 @@ __global__ void __launch_bounds__(NGI_BD_BLOCK, NGI_BD_WAVES) bdpt_kernel(Render
                         break;
                     }
                 }
+                // Read by the steps above only (as forget_vertex): the records hold them.
+                pv.gn = pv.n = ppv_p = f3(0.0f);
+                pv.prim = pv.type = 0;
+                pv.deg = false;
                 const uint32_t working = (uint32_t)__popcll(__ballot(!done));
                 if (working == 0) break;
                 if (__ballot(busy)) {

@@ -168,6 +168,14 @@ __device__ __forceinline__ bool light_begin(const RenderArgs& a, const Cam<R>& c
     return true;
 }
 
+// Forgets what only light_begin reads (as the path tracers' forget_vertex).
+template <typename R>
+__device__ __forceinline__ void forget_vertex(LightState<R>& ls) {
+    ls.s.gn = ls.s.n = ls.wi = V3<R>(R(0));
+    ls.s.degenerate = false;
+    ls.type = ls.prim = 0;
+}
+
 // light_end: the hit of the extension ray (h.leaf = -1 for a miss) and
 // Russian roulette.  Returns false when the path ends.
 template <typename R>

@@ -158,6 +158,7 @@ __global__ void __launch_bounds__(NGI_LT_BLOCK, (light_resume_waves<R, DIRECT, C
                 active = false;
             }
         }
+        forget_vertex(ls);
         const bool any = __ballot(active) != 0;
         if (QUEUE) {
             qcount += (uint32_t)__popcll(__ballot(pushed));   // at most q.cap - 65 + 64 (63 + 64 chunked)

@@ -181,7 +181,8 @@ __device__ __forceinline__ void shq_flush(const RenderArgs& a, const ShadowQueue
 // waits for its slowest ray once per drain instead of after every 64.  Starts
 // once the ring cannot take another 64 rays (or with any waiting, with `all`)
 // and returns with the queue empty.  Visits, tests and contributions are
-// those of shq_trace.
+// those of shq_trace.  For scenes with geometry (the kernels that drain are
+// those for at least NGI_CHUNKED_FEED_TRIS triangles).
 #ifndef NGI_SHQ_REFILL
 #define NGI_SHQ_REFILL 16
 #endif
@@ -198,6 +199,7 @@ __device__ __forceinline__ void shq_drain(const RenderArgs& a, const ShadowQueue
     int pixel = 0;
     uint32_t cur = 0, mask = 0;
     int sp = 0;
+    int32_t ref = 0;
     TraceCounters tc{0, 0};
     for (;;) {
         const unsigned long long idle = __ballot(!busy);
@@ -210,9 +212,9 @@ __device__ __forceinline__ void shq_drain(const RenderArgs& a, const ShadowQueue
                 shq_load<CT>(q, wave, head + rank, sr, C, pixel);
                 r = make_pre(sr);
                 tmax = sr.tmax;
-                cur = 0;
                 sp = 0;
-                mask = sc.num_tris ? NGI_TRAV8_FRESH : 0u;
+                mask = 0;
+                ref = 0;   // the root
                 busy = true;
                 cnt[CNT_SHADOW_RAYS]++;
             }
@@ -220,31 +222,41 @@ __device__ __forceinline__ void shq_drain(const RenderArgs& a, const ShadowQueue
             count -= take;
         }
         if (__ballot(busy) == 0) break;
-        // One node visit or leaf per lane, after at most one pop (Scene::Visible,
-        // rt.hpp:2251-2261; src/nanogi.cpp:700-706).
-        if (busy && mask == 0) {
-            if (sp == 0) {
-                busy = false;   // nothing in the way
-                film_add<FilmT>(a.film, pixel, C);
-            } else {
-                const uint32_t e = stk[(--sp) * stride];
-                cur = e >> 8;
-                mask = e & 0xffu;
-            }
-        }
+        // One node visit or leaf per lane, as in trav8_run: the next child is
+        // chosen, and its reference loaded, before the leaves are tested
+        // (Scene::Visible, rt.hpp:2251-2261; src/nanogi.cpp:700-706).
+        const bool leaf = busy && ref < 0;
+        const int32_t lref = ref;
+        bool more = busy;
+        Fetch f;
         if (busy) {
-            const int32_t ref = mask == NGI_TRAV8_FRESH ? 0 : next_child(sc, r, cur, mask);
-            mask &= mask - 1u;
-            const Fetch f = fetch_child(sc, ref);
-            if (ref < 0) {
-                TraceHit h;
-                if (leaf_test<true, COUNT>(sc, r, ref, f, NGI_EPS_F, tmax, h, tc)) busy = false;
-            } else {
+            f = fetch_child(sc, ref);
+            if (!leaf) {
                 if (mask) stk[(sp++) * stride] = (cur << 8) | mask;
                 cur = (uint32_t)ref;
                 mask = visit8<COUNT>(f, r, NGI_EPS_F, tmax, tc);
             }
+            if (mask == 0) {
+                if (sp == 0) {
+                    more = false;
+                } else {
+                    const uint32_t e = stk[(--sp) * stride];
+                    cur = e >> 8;
+                    mask = e & 0xffu;
+                }
+            }
+            if (more) {
+                ref = next_child(sc, r, cur, mask);
+                mask &= mask - 1u;
+            }
         }
+        bool occluded = false;
+        if (leaf) {
+            TraceHit h;
+            occluded = leaf_test<true, COUNT>(sc, r, lref, f, NGI_EPS_F, tmax, h, tc);
+        }
+        if (busy && !more && !occluded) film_add<FilmT>(a.film, pixel, C);   // nothing in the way
+        busy = more && !occluded;
     }
     if (COUNT) cnt[CNT_SH_NODES] += tc.nodes, cnt[CNT_SH_TRIS] += tc.tris;
 }
@@ -448,6 +460,18 @@ __device__ __forceinline__ void path_start(const RenderArgs& a, uint64_t id, con
     ps.s.n = V3<R>(R(0));
     ps.wi = V3<R>(R(0));
     ps.nv = 1;
+}
+
+// Forgets what only vertex_begin reads.  vertex_end and path_start write it
+// anew before the next one, so a lane whose extension ray is being traced need
+// not hold it; the kernels that resume traversals call this after
+// vertex_begin, which frees eleven registers per lane (twenty in FP64) for the
+// traversal loops (ptdirect at 96 VGPRs: 65 spilled without it, 31 with).
+template <typename R>
+__device__ __forceinline__ void forget_vertex(PathState<R>& ps) {
+    ps.s.gn = ps.s.n = ps.wi = V3<R>(R(0));
+    ps.s.degenerate = false;
+    ps.type = ps.prim = 0;
 }
 
 // One iteration of the vertex loop (src/nanogi.cpp:483-606 / 645-801) in two

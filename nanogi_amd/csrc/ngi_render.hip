@@ -236,6 +236,7 @@ __global__ void __launch_bounds__(NGI_MK_BLOCK, (resume_waves<R, DIRECT, CHUNKED
                 active = false;
             }
         }
+        forget_vertex(ps);
         const bool any = __ballot(active) != 0;
         if (QUEUE) {
             qcount += (uint32_t)__popcll(__ballot(pushed));   // at most q.cap - 65 + 64 (63 + 64 chunked)
