@@ -88,6 +88,7 @@ struct DevScene {
 // Owning host-side record of the device allocations of one scene.
 struct DeviceScene {
     int device = 0;
+    int cus = 0;   // compute units of the device
     hipStream_t stream = nullptr;
     DevScene view;
     std::vector<void*> allocs;

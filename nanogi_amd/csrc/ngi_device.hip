@@ -156,6 +156,9 @@ int device_prepare(HostScene& s) {
     }
     DeviceScene* d = new DeviceScene();
     s.dev = d;
+    int dev = 0;
+    NGI_HIP_CHECK(hipGetDevice(&dev));
+    NGI_HIP_CHECK(hipDeviceGetAttribute(&d->cus, hipDeviceAttributeMultiprocessorCount, dev));
     if (hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking) != hipSuccess) {
         d->stream = nullptr;
         return fail(NGI_ERR_DEVICE, "hipStreamCreate failed");
@@ -294,6 +297,96 @@ __global__ void __launch_bounds__(NGI_TRACE_BLOCK) trace_kernel(DevScene sc, con
     hits[i] = o;
 }
 
+// Many rays over the wide BVH: every wavefront takes `per_wave` consecutive
+// rays, and lanes whose rays have finished take the next ones as soon as
+// NGI_TRACE_REFILL of them are idle, so a wavefront waits for its slowest ray
+// once instead of after every 64 (one ray per lane left 11 of 64 lanes active
+// per VALU instruction on incoherent rays).  Visits, tests and results are
+// those of trace_bvh8; an iteration is as in trav8_run.  Bound by the latency
+// of the traversal's loads and by instruction issue.  Measured, us, one ray
+// per lane -> refills (1.5M / 6M rays; closest hit): sphere field with 1.8M
+// triangles 355 -> 314 / 1,070 -> 728, nave 296 -> 252 / 984 -> 809, a room of
+// 4,000 triangles 215 -> 154 / 705 -> 432, Cornell box 94 -> 92 / 304 -> 303;
+// any hit 1,064 -> 706 on 6M of the field's.  Refills of 8 or 24: the same
+// within 3%.
+#define NGI_TRACE_REFILL 16
+// Blocks per CU: 2 / 3 / 4 / 5 / 6 took 1,068 / 888 / 787 / 728 / 740 us for
+// the field's 6M rays and 409 / 337 / 342 / 314 / 325 for 1.5M.
+#define NGI_TRACE_WAVES 5
+// From two rays per lane on; with fewer a wavefront's last rays take as long
+// as all of them do (200,000 rays of the field: 162 us one ray per lane, 164
+// with refills; nave 86 and 103).
+#define NGI_TRACE_RAYS_PER_LANE 2
+template <bool ANY>
+__global__ void __launch_bounds__(NGI_TRACE_BLOCK, NGI_TRACE_WAVES) trace_refill_kernel(DevScene sc, const ngi_ray* __restrict__ rays, size_t n,
+                                                                                        ngi_hit* __restrict__ hits, size_t per_wave) {
+    extern __shared__ uint32_t stk[];   // sc.stack_entries x block
+    uint32_t* lds_stack = stk + threadIdx.x;
+    const uint32_t lane = __lane_id();
+    const size_t wave = (size_t)blockIdx.x * (NGI_TRACE_BLOCK / 64) + (threadIdx.x >> 6);
+    size_t next = wave * per_wave;   // wave-uniform; past n in the last wavefronts
+    const size_t end = next + per_wave < n ? next + per_wave : n;
+    bool busy = false;
+    size_t id = 0;
+    RayPre r;
+    float tmin = 0.0f;
+    Trav8 t;
+    int32_t ref = 0;
+    TraceCounters c{0, 0};
+    for (;;) {
+        const unsigned long long idle = __ballot(!busy);
+        const uint32_t nidle = (uint32_t)__popcll(idle);
+        if (next < end && (nidle >= NGI_TRACE_REFILL || nidle == 64u)) {
+            const size_t rank = (size_t)__popcll(idle & ((1ull << lane) - 1ull));
+            if (!busy && next + rank < end) {
+                id = next + rank;
+                const ngi_ray q = rays[id];
+                r = make_pre(TraceRay{q.o[0], q.o[1], q.o[2], q.d[0], q.d[1], q.d[2], q.tmin, q.tmax});
+                tmin = q.tmin;
+                trav8_begin(q.tmax, t);
+                t.mask = 0;
+                ref = 0;
+                busy = true;
+            }
+            next += nidle;
+        }
+        if (__ballot(busy) == 0) break;
+        const bool leaf = busy && ref < 0;
+        const int32_t lref = ref;
+        bool more = busy;
+        Fetch f;
+        if (busy) {
+            f = fetch_child(sc, ref);
+            if (!leaf) {
+                if (t.mask) lds_stack[(t.sp++) * NGI_TRACE_BLOCK] = (t.cur << 8) | t.mask;
+                t.cur = (uint32_t)ref;
+                t.mask = visit8<false>(f, r, tmin, t.h.t, c);
+            }
+            if (t.mask == 0) {
+                if (t.sp == 0) {
+                    more = false;
+                } else {
+                    const uint32_t e = lds_stack[(--t.sp) * NGI_TRACE_BLOCK];
+                    t.cur = e >> 8;
+                    t.mask = e & 0xffu;
+                }
+            }
+            if (more) {
+                ref = next_child(sc, r, t.cur, t.mask);
+                t.mask &= t.mask - 1u;
+            }
+        }
+        if (leaf && leaf_test<ANY, false>(sc, r, lref, f, tmin, t.h.t, t.h, c) && ANY) more = false;
+        if (busy && !more) {
+            ngi_hit o;
+            o.t = t.h.t, o.u = t.h.u, o.v = t.h.v;
+            o.tri = t.h.leaf < 0 ? NGI_MISS : __float_as_uint(sc.tris[3 * (size_t)t.h.leaf].w);
+            hits[id] = o;
+        }
+        busy = more;
+    }
+}
+
 int launch_trace(HostScene& s, const ngi_ray* d_rays, size_t n, ngi_hit* d_hits, int any_hit) {
     DeviceScene& d = *s.dev;
     if (n == 0) return NGI_OK;
@@ -308,6 +401,15 @@ int launch_trace(HostScene& s, const ngi_ray* d_rays, size_t n, ngi_hit* d_hits,
     const unsigned grid = (unsigned)((n + NGI_TRACE_BLOCK - 1) / NGI_TRACE_BLOCK);
     if (d.view.bvh_width == 8) {
         const size_t lds = (size_t)d.view.stack_entries * NGI_TRACE_BLOCK * 4;
+        const size_t lanes = (size_t)d.cus * NGI_TRACE_WAVES * NGI_TRACE_BLOCK;
+        if (n >= lanes * NGI_TRACE_RAYS_PER_LANE) {
+            const unsigned blocks = (unsigned)d.cus * NGI_TRACE_WAVES;
+            const size_t per = (n + (size_t)blocks * (NGI_TRACE_BLOCK / 64) - 1) / ((size_t)blocks * (NGI_TRACE_BLOCK / 64));
+            if (any_hit) trace_refill_kernel<true><<<blocks, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits, per);
+            else trace_refill_kernel<false><<<blocks, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits, per);
+            NGI_HIP_CHECK(hipGetLastError());
+            return NGI_OK;
+        }
         if (any_hit) trace_kernel<8, true><<<grid, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits);
         else trace_kernel<8, false><<<grid, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits);
     } else {

@@ -194,6 +194,26 @@ def test_trace_leaf_sizes(width, tris, leaf):
     assert np.array_equal(occluded, g["tri"] != ngi.MISS)
 
 
+@pytest.mark.parametrize("extra", [0, 1, 70001])
+@pytest.mark.parametrize("kind,detail", [(ngi.GEN_CORNELL, 0), (ngi.GEN_BATCH_ROOM, 3000)])
+def test_trace_many_rays_same_as_few(kind, detail, extra):
+    """Calls large enough for wavefronts that refill their lanes give each ray
+    what a small call gives it, at the smallest such size for 256 CUs and with
+    remainders of the wavefronts' shares."""
+    s = ngi.Scene.generate(kind, 2, 1.0, detail)
+    n = 256 * 5 * 256 * 2 + extra
+    rays = _random_rays([0.01] * 3, [0.99, 0.99, 2.0], n, 3)
+    rays["tmax"][::5] = 0.3
+    parts = np.array_split(np.arange(n), 5)
+    for any_hit in (False, True):
+        many = s.trace(rays, any_hit=any_hit)
+        few = np.concatenate([s.trace(rays[i], any_hit=any_hit) for i in parts])
+        if any_hit:
+            assert np.array_equal(many["tri"] == ngi.MISS, few["tri"] == ngi.MISS)
+        else:
+            assert np.array_equal(many.view(np.uint32), few.view(np.uint32))
+
+
 @pytest.mark.parametrize("scale", [1e-3, 1.0, 1e4])
 @pytest.mark.parametrize("length", [1e-6, 1.0, 1e6])
 def test_trace_scaled_scenes_and_directions(scale, length):
