@@ -521,7 +521,7 @@ int render_adjoint(ngi_scene* scene, const ngi_render_params& p, const double* d
     std::vector<void*> mem;
     auto cleanup = [&]() {
         (void)hipStreamSynchronize(str);
-        for (void* m : mem) (void)hipFree(m);
+        for (void* m : mem) workspace_free(m);
         S.destroy();
     };
     const int max_nv = (p.max_num_vertices < 0 || p.max_num_vertices > NGI_MAX_VERTICES) ? NGI_MAX_VERTICES : p.max_num_vertices;
@@ -571,7 +571,7 @@ int render_adjoint(ngi_scene* scene, const ngi_render_params& p, const double* d
     void *d_rp = nullptr, *d_rl = nullptr, *d_zm = nullptr;
 #define NGI_ADJ_ALLOC(ptr, bytes)                                   \
     do {                                                            \
-        hipError_t e_ = hipMalloc(&ptr, bytes);                     \
+        hipError_t e_ = workspace_alloc(&ptr, bytes);               \
         if (e_ != hipSuccess) {                                     \
             cleanup();                                              \
             return fail(NGI_ERR_OOM, "adjoint: hipMalloc failed");  \

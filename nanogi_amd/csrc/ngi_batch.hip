@@ -505,7 +505,7 @@ int Batch::refresh() {
 template <typename T>
 static int dev_alloc(T** ptr, size_t elems) {
     void* p = nullptr;
-    if (hipMalloc(&p, std::max<size_t>(elems, 1) * sizeof(T)) != hipSuccess) {
+    if (device_malloc(&p, std::max<size_t>(elems, 1) * sizeof(T)) != hipSuccess) {
         *ptr = nullptr;
         return fail(NGI_ERR_OOM, "batch: hipMalloc of %zu bytes failed", elems * sizeof(T));
     }
@@ -702,12 +702,10 @@ int Batch::get_film(int i, double* out) {
     if (i < 0 || i >= n()) return fail(NGI_ERR_INVALID_ARG, "scene index %d out of range", i);
     if (!rendered) return fail(NGI_ERR_INVALID_ARG, "the batch has not been rendered");
     const size_t m = film_off[i + 1] - film_off[i];
-    NGI_HIP_CHECK(hipMemcpyAsync(out, film + film_off[i], m * sizeof(double), hipMemcpyDeviceToHost, stream));
     NGI_HIP_CHECK(hipStreamSynchronize(stream));
     // W*H/N scaling (src/nanogi.cpp:434-437).
     const double scale = args[i].path_count ? (double)args[i].npix / (double)args[i].path_count : 0.0;
-    for (size_t k = 0; k < m; ++k) out[k] *= scale;
-    return NGI_OK;
+    return read_film(stream, film + film_off[i], true, m, scale, out);
 }
 
 int Batch::get_times(double* scene_ms, ngi_stats* stats) {

@@ -1,0 +1,224 @@
+// Kept device workspaces and the pinned read-back (ngi_mem.h).
+#include <string.h>
+
+#include <algorithm>
+#include <atomic>
+#include <mutex>
+#include <thread>
+#include <unordered_map>
+#include <vector>
+
+#include "ngi_dev.h"
+#include "ngi_mem.h"
+
+namespace ngi {
+
+#define NGI_KEPT_BYTES ((size_t)512 << 20)
+// The pinned buffer is a ring of NGI_PIN_SLOTS slots.
+#define NGI_PIN_SLOT ((size_t)1 << 20)
+#define NGI_PIN_SLOTS 16
+#define NGI_PIN_THREADS 8
+
+namespace {
+
+struct Workspaces {
+    std::mutex mu;
+    std::unordered_map<void*, size_t> size;   // of every block handed out or kept
+    std::vector<void*> kept;
+    size_t kept_bytes = 0;
+    int scenes = 0;
+
+    void trim() {
+        for (void* p : kept) {
+            size.erase(p);
+            (void)hipFree(p);
+        }
+        kept.clear();
+        kept_bytes = 0;
+    }
+};
+
+struct Pinned {
+    std::mutex mu;   // held while the buffer is in use
+    char* p = nullptr;
+    hipEvent_t done[NGI_PIN_SLOTS] = {};
+
+    bool ensure() {   // mu held
+        if (p) return true;
+        void* q = nullptr;
+        if (hipHostMalloc(&q, NGI_PIN_SLOT * NGI_PIN_SLOTS, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        for (hipEvent_t& e : done)
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                e = nullptr;
+                (void)hipHostFree(q);
+                return false;
+            }
+        p = static_cast<char*>(q);
+        return true;
+    }
+    void release() {   // mu held
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        for (hipEvent_t& e : done) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+    }
+};
+
+// Never destroyed: calls may come from other static destructors.
+Workspaces& workspaces() {
+    static Workspaces* w = new Workspaces();
+    return *w;
+}
+Pinned& pinned() {
+    static Pinned* p = new Pinned();
+    return *p;
+}
+
+}  // namespace
+
+hipError_t device_malloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    Workspaces& w = workspaces();
+    {
+        std::lock_guard<std::mutex> lock(w.mu);
+        w.trim();
+    }
+    return hipMalloc(p, bytes);
+}
+
+hipError_t workspace_alloc(void** p, size_t bytes) {
+    Workspaces& w = workspaces();
+    {
+        std::lock_guard<std::mutex> lock(w.mu);
+        size_t best = w.kept.size();
+        for (size_t i = 0; i < w.kept.size(); ++i) {
+            const size_t n = w.size[w.kept[i]];
+            // Not a block much larger than needed: it may be wanted as it is.
+            if (n >= bytes && n <= 2 * bytes + 65536 && (best == w.kept.size() || n < w.size[w.kept[best]])) best = i;
+        }
+        if (best < w.kept.size()) {
+            *p = w.kept[best];
+            w.kept_bytes -= w.size[*p];
+            w.kept.erase(w.kept.begin() + (long)best);
+            return hipSuccess;
+        }
+    }
+    const hipError_t e = device_malloc(p, bytes);
+    if (e != hipSuccess) return e;
+    std::lock_guard<std::mutex> lock(w.mu);
+    w.size[*p] = bytes;
+    return hipSuccess;
+}
+
+void workspace_free(void* p) {
+    if (!p) return;
+    Workspaces& w = workspaces();
+    std::lock_guard<std::mutex> lock(w.mu);
+    const auto it = w.size.find(p);
+    if (it == w.size.end()) return;
+    if (w.scenes > 0 && w.kept_bytes + it->second <= NGI_KEPT_BYTES) {
+        w.kept.push_back(p);
+        w.kept_bytes += it->second;
+        return;
+    }
+    w.size.erase(it);
+    (void)hipFree(p);
+}
+
+void resident_scenes(int delta) {
+    Workspaces& w = workspaces();
+    std::lock_guard<std::mutex> lock(w.mu);
+    w.scenes += delta;
+    if (w.scenes > 0) return;
+    w.trim();
+    Pinned& b = pinned();
+    std::lock_guard<std::mutex> pin(b.mu);
+    b.release();
+}
+
+PinnedBuffer::PinnedBuffer(size_t bytes) {
+    Pinned& b = pinned();
+    if (bytes > NGI_PIN_SLOT * NGI_PIN_SLOTS || !b.mu.try_lock()) return;
+    if (b.ensure()) p = b.p;
+    else b.mu.unlock();
+}
+PinnedBuffer::~PinnedBuffer() {
+    if (p) pinned().mu.unlock();
+}
+
+// The runtime's copy into pageable memory reads back 7 GB/s, on one thread
+// that mostly touches the caller's pages for the first time.  Here the device
+// fills the ring's slots (kernels write finished results straight into mapped
+// memory) while up to NGI_PIN_THREADS threads copy filled slots out.
+// Measured, whole calls, ms (with the kept workspaces): a 1280x720 film after
+// 1.2 ms of rendering 3.39 -> 2.17, a 1024x1024 film and its variance after
+// 32 ms 52.1 -> 34.1.
+int read_pinned(hipStream_t st, void* out, size_t bytes, const std::function<int(size_t, size_t, void*)>& emit) {
+    if (bytes == 0) return NGI_OK;
+    Pinned& b = pinned();
+    std::lock_guard<std::mutex> lock(b.mu);
+    if (!b.ensure()) return fail(NGI_ERR_OOM, "cannot pin %zu bytes of host memory", NGI_PIN_SLOT * NGI_PIN_SLOTS);
+    const size_t chunks = (bytes + NGI_PIN_SLOT - 1) / NGI_PIN_SLOT;
+    std::atomic<size_t> emitted{0}, taken{0}, copied[NGI_PIN_SLOTS];
+    for (auto& c : copied) c.store(0);   // chunks copied out of the slot so far
+    std::atomic<int> status{NGI_OK};
+    auto copy_one = [&]() -> bool {   // false: no chunk left
+        const size_t k = taken.fetch_add(1);
+        if (k >= chunks) return false;
+        while (emitted.load(std::memory_order_acquire) <= k) {
+            if (status.load() != NGI_OK) return false;
+            std::this_thread::yield();
+        }
+        const size_t slot = k % NGI_PIN_SLOTS, at = k * NGI_PIN_SLOT;
+        if (hipEventSynchronize(b.done[slot]) != hipSuccess) {
+            status.store(NGI_ERR_DEVICE);
+            return false;
+        }
+        memcpy(static_cast<char*>(out) + at, b.p + slot * NGI_PIN_SLOT, std::min(NGI_PIN_SLOT, bytes - at));
+        copied[slot].fetch_add(1, std::memory_order_release);
+        return true;
+    };
+    std::vector<std::thread> helpers;
+    const size_t want = std::min<size_t>({chunks - 1, NGI_PIN_THREADS - 1, std::max(1u, std::thread::hardware_concurrency()) - 1});
+    try {
+        helpers.reserve(want);
+        for (size_t i = 0; i < want; ++i)
+            helpers.emplace_back([&] {
+                while (copy_one()) {
+                }
+            });
+    } catch (...) {   // no more threads: those there are do it
+    }
+    for (size_t k = 0; k < chunks && status.load() == NGI_OK; ++k) {
+        const size_t slot = k % NGI_PIN_SLOTS, at = k * NGI_PIN_SLOT;
+        while (copied[slot].load(std::memory_order_acquire) < k / NGI_PIN_SLOTS) {   // the slot's previous chunk
+            if (status.load() != NGI_OK) break;
+            if (helpers.empty()) (void)copy_one();
+            else std::this_thread::yield();
+        }
+        if (status.load() != NGI_OK) break;
+        const int s = emit(at, std::min(NGI_PIN_SLOT, bytes - at), b.p + slot * NGI_PIN_SLOT);
+        if (s != NGI_OK) status.store(s);
+        else if (hipEventRecord(b.done[slot], st) != hipSuccess) status.store(NGI_ERR_DEVICE);
+        else emitted.store(k + 1, std::memory_order_release);
+    }
+    while (status.load() == NGI_OK && copy_one()) {
+    }
+    for (std::thread& t : helpers) t.join();
+    const int s = status.load();
+    if (s != NGI_OK) {
+        (void)hipStreamSynchronize(st);   // nothing writes the buffer once it is let go
+        return s == NGI_ERR_DEVICE ? fail(NGI_ERR_DEVICE, "reading results back failed") : s;
+    }
+    return NGI_OK;
+}
+
+}  // namespace ngi

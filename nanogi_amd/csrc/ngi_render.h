@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "ngi_mem.h"
 #include "ngi_path.h"
 
 namespace ngi {
@@ -63,11 +64,11 @@ struct LaneMem {
         if (fixed) return fail(NGI_ERR_INVALID_ARG, "launch needs %zu bytes of per-lane records, the fixed buffer holds %zu", n, *bytes);
         if (*ptr) {
             NGI_HIP_CHECK(hipStreamSynchronize(stream));
-            NGI_HIP_CHECK(hipFree(*ptr));
+            workspace_free(*ptr);
         }
         *ptr = nullptr;
         *bytes = 0;
-        if (hipMalloc(ptr, n) != hipSuccess) {
+        if (workspace_alloc(ptr, n) != hipSuccess) {
             *ptr = nullptr;
             (void)hipGetLastError();   // a later call's launch check must not see this refusal
             return fail(NGI_ERR_OOM, "cannot allocate %zu bytes of per-lane records", n);
@@ -96,6 +97,10 @@ inline bool persistent_only(int renderer) { return is_light_tracer(renderer) || 
 // precision, engine, roulette, vertex cap, sensor).
 int check_render_params(const ngi_scene* sc, const ngi_render_params& p);
 
+// n film values (FP64, or FP32), scaled, into host memory; the caller has
+// waited for the work that writes the film.
+int read_film(hipStream_t st, const void* film, bool film64, size_t n, double scale, double* out);
+
 struct Session {
     ngi_scene* scene = nullptr;
     ngi_render_params p;
@@ -121,6 +126,7 @@ struct Session {
     int ensure_device();
     int init(ngi_scene* sc, const ngi_render_params& pp);
     int reset();
+    int clear();   // reset without waiting
     void destroy();
     int zero(void* p, size_t n_elems, bool f64);
     RenderArgs args(void* target_film) const;

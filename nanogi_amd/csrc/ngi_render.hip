@@ -11,6 +11,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "ngi_mem.h"
 #include "ngi_path.h"
 #include "ngi_render.h"
 
@@ -356,6 +357,36 @@ __global__ void fold_batch(const FilmT* __restrict__ batch, double scale, double
     film[i] += (FilmT)b;
 }
 
+// The film as ngi_session_get_film returns it: scaled by W*H/N
+// (src/nanogi.cpp:434-437), in FP64.
+template <typename FilmT>
+__global__ void film_out(const FilmT* __restrict__ film, double scale, double* __restrict__ out, size_t n) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = (double)film[i] * scale;
+}
+
+int read_film(hipStream_t st, const void* film, bool film64, size_t n, double scale, double* out) {
+    return read_pinned(st, out, n * 8, [&](size_t at, size_t bytes, void* dst) {
+        const size_t i0 = at / 8, m = bytes / 8;
+        const unsigned grid = (unsigned)((m + 255) / 256);
+        double* o = reinterpret_cast<double*>(dst);
+        if (film64) film_out<double><<<grid, 256, 0, st>>>(reinterpret_cast<const double*>(film) + i0, scale, o, m);
+        else film_out<float><<<grid, 256, 0, st>>>(reinterpret_cast<const float*>(film) + i0, scale, o, m);
+        NGI_HIP_CHECK(hipGetLastError());
+        return (int)NGI_OK;
+    });
+}
+
+// Variance of the mean of k batch films from their first and second moments.
+__global__ void variance_out(const double* __restrict__ m1, const double* __restrict__ m2, double k, double* __restrict__ out, size_t n) {
+#pragma clang fp contract(off)
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double mean = m1[i] / k;
+    const double sv = (m2[i] - k * mean * mean) / (k - 1.0);   // sample variance of batch means
+    out[i] = (sv > 0 ? sv : 0.0) / k;
+}
+
 template <typename FilmT>
 __global__ void zero_kernel(FilmT* p, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -410,12 +441,17 @@ int Session::init(ngi_scene* sc, const ngi_render_params& pp) {
     film64 = p.precision != NGI_PRECISION_FP32_ALL;
     npix = (uint32_t)p.width * (uint32_t)p.height;
     const size_t fb = (size_t)npix * 3 * (film64 ? 8 : 4);
-    NGI_HIP_CHECK(hipMalloc(&film, fb));
-    NGI_HIP_CHECK(hipMalloc(&counters, CNT_N * sizeof(unsigned long long)));
-    return reset();
+    NGI_HIP_CHECK(workspace_alloc(&film, fb));
+    NGI_HIP_CHECK(workspace_alloc(&counters, CNT_N * sizeof(unsigned long long)));
+    return clear();   // what follows is enqueued behind it
 }
 
 int Session::reset() {
+    const int st = clear();
+    return st ? st : sync();
+}
+
+int Session::clear() {
     paths_done = 0;
     samples_done = 0;
     batches = 0;
@@ -426,13 +462,12 @@ int Session::reset() {
         if ((st = zero(m1, (size_t)npix * 3, true))) return st;
         if ((st = zero(m2, (size_t)npix * 3, true))) return st;
     }
-    if ((st = zero(counters, CNT_N, true))) return st;   // 64-bit words
-    return sync();
+    return zero(counters, CNT_N, true);   // 64-bit words
 }
 
 void Session::destroy() {
     if (scene && scene->dev) (void)hipStreamSynchronize(stream());
-    for (void* q : {film, counters, m1, m2, batch, next_path, lane_mem}) if (q) (void)hipFree(q);
+    for (void* q : {film, counters, m1, m2, batch, next_path, lane_mem}) workspace_free(q);
     film = counters = m1 = m2 = batch = next_path = lane_mem = nullptr;
     lane_bytes = 0;
     release_engine();
@@ -520,7 +555,7 @@ int Session::render_into(void* target, int spp) {
         st = render_wavefront(target, total);
     } else if (p.engine == NGI_ENGINE_PERSISTENT || persistent_only(p.renderer)) {
         // The light tracers and bdpt always run on the persistent engine.
-        if (!next_path) NGI_HIP_CHECK(hipMalloc(&next_path, sizeof(unsigned long long)));
+        if (!next_path) NGI_HIP_CHECK(workspace_alloc(&next_path, sizeof(unsigned long long)));
         if ((st = zero(next_path, 1, true))) return st;
         RenderArgs a = args(target);
         a.sample_base = samples_done;
@@ -576,9 +611,9 @@ int Session::render(int spp) { return render_into(film, spp); }
 int Session::render_batch(int spp) {
     const size_t n = (size_t)npix * 3;
     if (!m1) {
-        NGI_HIP_CHECK(hipMalloc(&m1, n * 8));
-        NGI_HIP_CHECK(hipMalloc(&m2, n * 8));
-        NGI_HIP_CHECK(hipMalloc(&batch, n * (film64 ? 8 : 4)));
+        NGI_HIP_CHECK(workspace_alloc(&m1, n * 8));
+        NGI_HIP_CHECK(workspace_alloc(&m2, n * 8));
+        NGI_HIP_CHECK(workspace_alloc(&batch, n * (film64 ? 8 : 4)));
         int st = zero(m1, n, true);
         if (!st) st = zero(m2, n, true);
         if (st) return st;
@@ -601,27 +636,22 @@ int Session::get_film(double* out, double* var) {
     if (st) return st;
     const size_t n = (size_t)npix * 3;
     const double scale = paths_done ? (double)npix / (double)paths_done : 0.0;
+    // Both are finished on the device, in FP64, on their way out.
     if (out) {
-        if (film64) {
-            NGI_HIP_CHECK(hipMemcpy(out, film, n * 8, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < n; ++i) out[i] *= scale;
-        } else {
-            std::vector<float> tmp(n);
-            NGI_HIP_CHECK(hipMemcpy(tmp.data(), film, n * 4, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < n; ++i) out[i] = (double)tmp[i] * scale;
-        }
+        st = read_film(stream(), film, film64, n, scale, out);
+        if (st) return st;
     }
     if (var) {
         if (!m1 || batches < 2) return fail(NGI_ERR_INVALID_ARG, "variance needs at least two batches (ngi_session_render_batch)");
-        std::vector<double> a(n), b(n);
-        NGI_HIP_CHECK(hipMemcpy(a.data(), m1, n * 8, hipMemcpyDeviceToHost));
-        NGI_HIP_CHECK(hipMemcpy(b.data(), m2, n * 8, hipMemcpyDeviceToHost));
-        const double k = (double)batches;
-        for (size_t i = 0; i < n; ++i) {
-            const double mean = a[i] / k;
-            const double sv = (b[i] - k * mean * mean) / (k - 1.0);   // sample variance of batch means
-            var[i] = (sv > 0 ? sv : 0.0) / k;
-        }
+        st = read_pinned(stream(), var, n * 8, [&](size_t at, size_t bytes, void* dst) {
+            const size_t i0 = at / 8, m = bytes / 8;
+            variance_out<<<(unsigned)((m + 255) / 256), 256, 0, stream()>>>(reinterpret_cast<const double*>(m1) + i0,
+                                                                            reinterpret_cast<const double*>(m2) + i0, (double)batches,
+                                                                            reinterpret_cast<double*>(dst), m);
+            NGI_HIP_CHECK(hipGetLastError());
+            return (int)NGI_OK;
+        });
+        if (st) return st;
     }
     return NGI_OK;
 }
@@ -630,7 +660,11 @@ int Session::get_stats(ngi_stats* out) {
     int st = sync();
     if (st) return st;
     unsigned long long c[CNT_N];
-    NGI_HIP_CHECK(hipMemcpy(c, counters, sizeof(c), hipMemcpyDeviceToHost));
+    st = read_pinned(stream(), c, sizeof(c), [&](size_t, size_t bytes, void* dst) {
+        NGI_HIP_CHECK(hipMemcpyAsync(dst, counters, bytes, hipMemcpyDeviceToHost, stream()));
+        return (int)NGI_OK;
+    });
+    if (st) return st;
     *out = stats;
     out->samples = (int64_t)c[CNT_SAMPLES];
     out->extension_rays = (int64_t)c[CNT_EXT_RAYS];

@@ -315,14 +315,13 @@ static int run_wf2(Session& S, WavefrontState& W, void* target, uint64_t total, 
 static int wf_alloc(WavefrontState& W, uint32_t cap) {
     W.capacity = cap;
     for (int k = 0; k < 2; ++k) {
-        NGI_HIP_CHECK(hipMalloc(&W.ray[k], (size_t)cap * 32));
-        NGI_HIP_CHECK(hipMalloc(&W.st[k], (size_t)cap * 32));
+        NGI_HIP_CHECK(workspace_alloc(&W.ray[k], (size_t)cap * 32));
+        NGI_HIP_CHECK(workspace_alloc(&W.st[k], (size_t)cap * 32));
     }
-    NGI_HIP_CHECK(hipMalloc(&W.hit, (size_t)cap * 16));
-    NGI_HIP_CHECK(hipMalloc(&W.shadow, (size_t)cap * 2 * 48));
-    NGI_HIP_CHECK(hipMalloc(&W.counts, 4 * sizeof(uint32_t)));
+    NGI_HIP_CHECK(workspace_alloc(&W.hit, (size_t)cap * 16));
+    NGI_HIP_CHECK(workspace_alloc(&W.shadow, (size_t)cap * 2 * 48));
+    NGI_HIP_CHECK(workspace_alloc(&W.counts, 4 * sizeof(uint32_t)));
     NGI_HIP_CHECK(hipHostMalloc((void**)&W.host_counts, 4 * sizeof(uint32_t), hipHostMallocDefault));
-    NGI_HIP_CHECK(hipMemset(W.counts, 0, 4 * sizeof(uint32_t)));
     return NGI_OK;
 }
 
@@ -345,8 +344,11 @@ int Session::render_wavefront(void* target, uint64_t total) {
     while (!wf) {
         wf = new WavefrontState();
         const uint32_t cap = std::max<uint32_t>(p.paths_in_flight > 0 ? (uint32_t)p.paths_in_flight : def, 256);
-        const int st = wf_alloc(*wf, cap);
-        if (!st) break;
+        int st = wf_alloc(*wf, cap);
+        if (!st) {
+            if ((st = zero(wf->counts, 2, true))) return st;   // four 32-bit words, on the session's stream
+            break;
+        }
         release_engine();          // frees what was allocated; wf = nullptr
         (void)hipGetLastError();   // the refused allocation must not fail the next launch check
         if (st != NGI_ERR_OOM || p.paths_in_flight > 0 || cap <= (1u << 16)) return st;
@@ -362,12 +364,12 @@ int Session::render_wavefront(void* target, uint64_t total) {
 void Session::release_engine() {
     if (!wf) return;
     for (int k = 0; k < 2; ++k) {
-        if (wf->ray[k]) (void)hipFree(wf->ray[k]);
-        if (wf->st[k]) (void)hipFree(wf->st[k]);
+        if (wf->ray[k]) workspace_free(wf->ray[k]);
+        if (wf->st[k]) workspace_free(wf->st[k]);
     }
-    if (wf->hit) (void)hipFree(wf->hit);
-    if (wf->shadow) (void)hipFree(wf->shadow);
-    if (wf->counts) (void)hipFree(wf->counts);
+    if (wf->hit) workspace_free(wf->hit);
+    if (wf->shadow) workspace_free(wf->shadow);
+    if (wf->counts) workspace_free(wf->counts);
     if (wf->host_counts) (void)hipHostFree(wf->host_counts);
     delete wf;
     wf = nullptr;

@@ -1,0 +1,98 @@
+"""Kept device workspaces and the pinned read-back (ngi_mem): films of every
+size come back whole, one call's leftovers never show in the next, and
+threads may render at once.
+"""
+import threading
+
+import numpy as np
+import pytest
+
+import nanogi_amd as ngi
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _params(renderer, w, h, spp=1, **kw):
+    return ngi.default_params(renderer=renderer, width=w, height=h, sampling=ngi.SAMPLING_PER_PIXEL, spp=spp, max_num_vertices=5,
+                              rr_depth=3, seed=11, **kw)
+
+
+# The read-back goes in slots of 1 MiB (43,690.7 pixels) through a ring of 16.
+@pytest.mark.parametrize("w,h", [(1, 1), (257, 170), (43691, 1), (1024, 700)])
+@pytest.mark.parametrize("precision", [ngi.PRECISION_FP32_FP64ACC, ngi.PRECISION_FP32_ALL])
+def test_film_sizes_against_oracle(w, h, precision):
+    s = ngi.Scene.generate(ngi.GEN_CORNELL, 1, 1.0)
+    p = _params("ptdirect", w, h, precision=precision)
+    film, st = ngi.render(s, p)
+    ref = oracle.render(s, p)
+    assert st["samples"] == w * h
+    rel = np.abs(film - ref).max(axis=2) / (np.abs(ref).max(axis=2) + 1e-3)
+    assert (rel < 2e-4).mean() >= 0.97
+
+
+def test_variance_is_that_of_the_batches():
+    s = ngi.Scene.generate(ngi.GEN_CORNELL, 1, 1.0)
+    p = _params("pt", 300, 260)
+    batches = []
+    for k in range(3):
+        se = ngi.Session(s, p)
+        if k:
+            se.render(k)        # samples 0..k-1, then the batch's own
+        before = se.film() * k
+        se.render(1)
+        batches.append(se.film() * (k + 1) - before)
+        se.close()
+    se = ngi.Session(s, p)
+    for _ in range(3):
+        se.render_batch(1)
+    film, var = se.film(variance=True)
+    b = np.stack(batches)
+    # FP64 sums of FP32 contributions: differences of films cost about 1e-15 of the largest value.
+    tol = 1e-12 * max(1.0, np.abs(b).max()) ** 2
+    assert np.abs(film - b.mean(axis=0)).max() <= tol
+    assert np.abs(var - b.var(axis=0, ddof=1) / 3).max() <= tol
+
+
+def test_leftovers_of_other_calls_do_not_show():
+    a = ngi.Scene.generate(ngi.GEN_CORNELL, 1, 1.0)
+    b = ngi.Scene.generate(ngi.GEN_NAVE, 2, 1.0)   # large enough for the 512-record shadow rings
+    jobs = []
+    for scene in (a, b):
+        for renderer in ("pt", "ptdirect", "ltdirect", "bdpt"):
+            for w, h, spp in ((96, 64, 2), (31, 17, 1)):
+                jobs.append((scene, _params(renderer, w, h, spp)))
+        jobs.append((scene, _params("ptdirect", 64, 48, 2, engine=ngi.ENGINE_WAVEFRONT)))
+    first = [ngi.render(s, p)[0] for s, p in jobs]
+    for i in np.random.default_rng(0).permutation(len(jobs)):
+        again = ngi.render(*jobs[i])[0]
+        assert np.abs(again - first[i]).max() <= 1e-9 * max(1.0, np.abs(first[i]).max())
+    g = np.random.default_rng(1).normal(size=(48, 64, 3))
+    p = _params("ptdirect", 64, 48, 4)
+    gR, gL, _ = ngi.render_adjoint(a, p, g)
+    ngi.render(b, _params("pt", 200, 100))
+    gR2, gL2, _ = ngi.render_adjoint(a, p, g)
+    assert np.allclose(gR, gR2, rtol=1e-9, atol=1e-12) and np.allclose(gL, gL2, rtol=1e-9, atol=1e-12)
+
+
+def test_threads_render_at_once():
+    sizes = [(40, 30), (300, 200), (640, 480), (17, 9)]
+    scenes = [ngi.Scene.generate(ngi.GEN_BATCH_ROOM, 20 + i, 1.0, 200) for i in range(4)]
+    params = [_params("ptdirect", w, h, 2) for w, h in sizes]
+    rays = ngi.make_rays(np.full((50, 3), 0.5), np.random.default_rng(3).normal(size=(50, 3)))
+    want = [(ngi.render(s, p)[0], s.trace(rays)) for s, p in zip(scenes, params)]
+    bad = []
+
+    def work(i):
+        for _ in range(6):
+            film = ngi.render(scenes[i], params[i])[0]
+            hits = scenes[i].trace(rays)
+            if np.abs(film - want[i][0]).max() > 1e-9 * np.abs(want[i][0]).max() or not np.array_equal(hits, want[i][1]):
+                bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
