@@ -286,3 +286,21 @@ def test_reduced_room_batch_against_the_oracle():
         assert frac >= 0.98, (i, s.num_triangles, frac)
         np.testing.assert_allclose(f.reshape(-1, 3).mean(0), o.reshape(-1, 3).mean(0), rtol=2e-3, err_msg=str(i))
     b.close()
+
+
+@pytest.mark.parametrize("scenes,chunk", [(1, 1 << 24), (1, 7), (3, 64), (33, 1 << 20), (40, 100)])
+def test_batch_chunk_counts(scenes, chunk):
+    """Fewer chunks than groups of wavefronts, one per scene, and many more:
+    every path is rendered exactly once."""
+    sc = [ngi.Scene.generate(ngi.GEN_BATCH_ROOM, 50 + i, 1.0, 12 + 5 * i) for i in range(scenes)]
+    ps = [_p("ptdirect", 9 + i % 5, 7 + i % 3, 2 + i % 4, 5, 3, seed=i + 1) for i in range(scenes)]
+    b = ngi.Batch(sc, ps, ngi.batch_opts(block_size=128, blocks_per_cu=2, chunk_paths=chunk))
+    for frame in (0, 0):
+        b.render(frame)
+        b.sync()
+        for i in range(scenes):
+            one, _ = ngi.render(sc[i], ps[i])
+            assert np.abs(b.film(i) - one).max() <= 1e-9 * max(1.0, np.abs(one).max())
+        ms, st = b.times()
+        assert st["samples"] == sum(p.width * p.height * p.spp for p in ps) and (ms > 0).all()
+    b.close()
