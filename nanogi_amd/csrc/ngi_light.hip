@@ -132,10 +132,10 @@ __global__ void __launch_bounds__(NGI_LT_BLOCK, (light_resume_waves<R, DIRECT, C
         if (active && !busy)
             active = light_end<R>(a, prims, ls, parked_dir_r<NGI_LT_BLOCK, R>(pk), parked_urr_r<NGI_LT_BLOCK, R>(pk), parked_hit<NGI_LT_BLOCK>(pk));
         if (!feed.done()) {
-            const unsigned long long need = __ballot(!active);
-            if (need && ((uint32_t)__popcll(need) >= (CHUNKED ? 1u : (uint32_t)NGI_LT_PATH_REFILL) || need == ~0ull)) {
+            const unsigned long long need = __ballot(!active && __lane_id() < a.path_lanes);
+            if (need && ((uint32_t)__popcll(need) >= (CHUNKED ? 1u : (uint32_t)NGI_LT_PATH_REFILL) || __ballot(active) == 0)) {
                 const unsigned long long id = feed.take<CHUNKED>(next, a.path_count, need, a.path_chunk);
-                if (!active && id != ~0ull) {
+                if (id != ~0ull) {
                     cnt[CNT_SAMPLES]++;
                     active = light_start<R>(a, a.path_begin + id, ls);
                 }
@@ -202,15 +202,21 @@ static int launch_lt(const RenderArgs& a, unsigned long long* next, LaneMem mem,
     auto kern = resume ? (a.path_chunk ? light_resume_kernel<R, FilmT, DIRECT, COUNT, true> : light_resume_kernel<R, FilmT, DIRECT, COUNT, false>)
                        : (a.path_chunk ? light_kernel<R, FilmT, DIRECT, WIDTH, COUNT, true> : light_kernel<R, FilmT, DIRECT, WIDTH, COUNT, false>);
     unsigned grid = 0;
-    int s = persistent_grid(reinterpret_cast<const void*>(kern), NGI_LT_BLOCK, lds, a.path_count, ln, &grid);
+    int64_t full = 0;
+    int s = persistent_grid(reinterpret_cast<const void*>(kern), NGI_LT_BLOCK, lds, a.path_count, Lanes{ln.want, &full}, &grid);
+    if (ln.full) *ln.full = full;
     if (s || !grid) return s;
+    RenderArgs b = a;
+    const size_t rec = (size_t)ShqWords<R>::value * sizeof(float4);
+    const bool queue = DIRECT && (std::is_same<R, float>::value || (resume && !a.path_chunk));
+    const bool rings = !queue || !mem.fixed || rec * 2 * grid * (NGI_LT_BLOCK / 64) * NGI_SHQ <= *mem.bytes;
+    persistent_feed(b, NGI_LT_BLOCK, (uint64_t)full, resume && rings && (ln.want == 0 || a.path_count <= (uint64_t)ln.want), &grid);
     ShadowQueue q;
     q.waves = grid * (NGI_LT_BLOCK / 64);
     q.rec = nullptr;
-    if (DIRECT && (std::is_same<R, float>::value || (resume && !a.path_chunk))) {
+    if (queue) {
         // Longer rings for the refilling drains; a caller-owned buffer gets
         // the longest ring it holds, and as many blocks as it has rings for.
-        const size_t rec = (size_t)ShqWords<R>::value * sizeof(float4);
         if (resume && !a.path_chunk) {
             q.cap = NGI_SHQ_LONG;
             while (mem.fixed && q.cap > NGI_SHQ && rec * q.waves * q.cap > *mem.bytes) q.cap >>= 1;
@@ -223,7 +229,7 @@ static int launch_lt(const RenderArgs& a, unsigned long long* next, LaneMem mem,
         if ((s = mem.reserve(rec * q.waves * q.cap))) return s;
         q.rec = reinterpret_cast<float4*>(*mem.ptr);
     }
-    kern<<<grid, NGI_LT_BLOCK, lds, st>>>(a, next, q);
+    kern<<<grid, NGI_LT_BLOCK, lds, st>>>(b, next, q);
     NGI_HIP_CHECK(hipGetLastError());
     return NGI_OK;
 }

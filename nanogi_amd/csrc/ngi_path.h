@@ -41,6 +41,7 @@ struct RenderArgs {
     uint32_t seed, stream_id;
     unsigned long long* counters;   // CNT_N entries or null
     uint32_t path_chunk;            // persistent engines: path ids per counter atomic (0 = exactly the ids needed)
+    uint32_t path_lanes;            // resumable kernels: lanes of a wavefront that take paths (32 or 64)
 };
 
 template <typename R> __device__ __forceinline__ R unif(uint32_t x);

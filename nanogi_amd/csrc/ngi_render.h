@@ -50,6 +50,27 @@ inline int persistent_grid(const void* kern, int block, size_t lds, uint64_t pat
     return NGI_OK;
 }
 
+// Feed of a persistent launch of `grid` blocks of which the device holds
+// `full` lanes.  A chunk (RenderArgs::path_chunk) is at most a quarter of a
+// wavefront's share of the paths: chunks of 128 gave a launch of one path per
+// lane to half of its wavefronts, twice 64 paths one after the other (58,000
+// paths in a 2k-triangle room: 375 -> 252 us).  A launch that leaves half of
+// the device's lanes unused runs (`spread`, resumable kernels) on twice the
+// wavefronts with 32 paths each, which wait for the slowest of 32 rays instead
+// of 64 (whole ngi_render calls, us: 14,400 paths on the nave 421 -> 357, pt
+// 317 -> 280; 28,800 on a 90k-triangle sphere field 424 -> 399; 58,000 in the
+// room 343 -> 334; with 16 paths each 401, 321, 387, 391: more wavefronts
+// issue more instructions for the same paths).
+inline void persistent_feed(RenderArgs& a, int block, uint64_t full, bool spread, unsigned* grid) {
+    const uint64_t blocks = (2 * a.path_count + block - 1) / block;
+    if (spread && blocks * block <= full) {
+        a.path_lanes = 32;
+        *grid = (unsigned)blocks;
+    }
+    const uint64_t waves = (uint64_t)*grid * (block / 64);
+    if (a.path_chunk) a.path_chunk = (uint32_t)std::min<uint64_t>(a.path_chunk, std::max<uint64_t>(1, a.path_count / (4 * waves)));
+}
+
 // Device scratch owned by a session and grown on demand (per-lane bdpt
 // subpath records, per-wavefront shadow queues).  Growing waits for the
 // session's stream first: an earlier launch may still be using the buffer.

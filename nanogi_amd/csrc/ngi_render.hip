@@ -145,6 +145,9 @@ __global__ void __launch_bounds__(NGI_MK_BLOCK, CHUNKED && DIRECT ? NGI_PK_WAVES
 // lanes).  With paths refilled 16 at a time (nave / room): diffuse keep 10:
 // 739 / 1,447, 12: 743 / 1,470, 16: 748 / 1,496, 20: 749 / 1,505, 24: 746 /
 // 1,504; glossy keep 6 / 8 / 10 on the sphere field: 1,861 / 1,863 / 1,867.
+// Once the launch has no paths left a quarter of the busy lanes wait: the
+// wavefront's last paths follow one another less (58,000 paths in a 2k-triangle
+// room: 258 us with none left waiting, 252 with a quarter, 267 with half).
 //
 // FP64 shading (R = double) parks its direction and roulette number in FP64
 // and queues its shadow rays with FP64 contributions (four float4s per
@@ -210,10 +213,10 @@ __global__ void __launch_bounds__(NGI_MK_BLOCK, (resume_waves<R, DIRECT, CHUNKED
             active = vertex_end<R, FilmT, DIRECT>(a, prims, ps, parked_dir_r<NGI_MK_BLOCK, R>(pk), parked_urr_r<NGI_MK_BLOCK, R>(pk),
                                                   parked_hit<NGI_MK_BLOCK>(pk));
         if (!feed.done()) {
-            const unsigned long long need = __ballot(!active);
-            if (need && ((uint32_t)__popcll(need) >= (CHUNKED ? 1u : (uint32_t)NGI_PK_PATH_REFILL) || need == ~0ull)) {
+            const unsigned long long need = __ballot(!active && __lane_id() < a.path_lanes);
+            if (need && ((uint32_t)__popcll(need) >= (CHUNKED ? 1u : (uint32_t)NGI_PK_PATH_REFILL) || __ballot(active) == 0)) {
                 const unsigned long long id = feed.take<CHUNKED>(next, a.path_count, need, a.path_chunk);
-                if (!active && id != ~0ull) {
+                if (id != ~0ull) {
                     path_start<R>(a, a.path_begin + id, cam, ps);
                     cnt[CNT_SAMPLES]++;
                     active = true;
@@ -252,7 +255,8 @@ __global__ void __launch_bounds__(NGI_MK_BLOCK, (resume_waves<R, DIRECT, CHUNKED
             // Lanes without a ray load and store back what they parked last.
             Trav8 tv = parked_trav<NGI_MK_BLOCK>(pk);
             const RayPre r = make_pre(extension_ray(ps, parked_dir_r<NGI_MK_BLOCK, R>(pk)));
-            const int keep = __builtin_amdgcn_readfirstlane(feed.done() ? 0 : (a.sc.any_glossy ? NGI_PK_KEEP : NGI_PK_KEEP_DIFFUSE));
+            const int keep = __builtin_amdgcn_readfirstlane(
+                feed.done() ? (int)__popcll(__ballot(busy)) / 4 : (a.sc.any_glossy ? NGI_PK_KEEP : NGI_PK_KEEP_DIFFUSE));
             trav8_run<COUNT>(a.sc, r, NGI_EPS_F, tv, busy, keep, tc, ext_stk, NGI_MK_BLOCK);
             park_trav<NGI_MK_BLOCK>(pk, tv);
         }
@@ -293,16 +297,22 @@ static int launch_pk(const RenderArgs& a, unsigned long long* next, LaneMem mem,
                        : (a.path_chunk ? persistent_kernel<R, FilmT, DIRECT, WIDTH, COUNT, true>
                                        : persistent_kernel<R, FilmT, DIRECT, WIDTH, COUNT, false>);
     unsigned grid = 0;
-    int s = persistent_grid(reinterpret_cast<const void*>(kern), NGI_MK_BLOCK, lds, a.path_count, ln, &grid);
+    int64_t full = 0;
+    int s = persistent_grid(reinterpret_cast<const void*>(kern), NGI_MK_BLOCK, lds, a.path_count, Lanes{ln.want, &full}, &grid);
+    if (ln.full) *ln.full = full;
     if (s || !grid) return s;
+    RenderArgs b = a;
+    const size_t rec = (size_t)ShqWords<R>::value * sizeof(float4);
+    const bool queue = DIRECT && (std::is_same<R, float>::value || (resume && !a.path_chunk));
+    const bool rings = !queue || !mem.fixed || rec * 2 * grid * (NGI_MK_BLOCK / 64) * NGI_SHQ <= *mem.bytes;
+    persistent_feed(b, NGI_MK_BLOCK, (uint64_t)full, resume && rings && (ln.want == 0 || a.path_count <= (uint64_t)ln.want), &grid);
     ShadowQueue q;
     q.waves = grid * (NGI_MK_BLOCK / 64);
     q.rec = nullptr;
-    if (DIRECT && (std::is_same<R, float>::value || (resume && !a.path_chunk))) {
+    if (queue) {
         // Longer rings for the refilling drains; a caller-owned buffer gets
         // the longest ring it holds, and as many blocks as it has rings for
         // (the persistent grid takes every path with fewer blocks too).
-        const size_t rec = (size_t)ShqWords<R>::value * sizeof(float4);
         if (resume && !a.path_chunk) {
             q.cap = NGI_SHQ_LONG;
             while (mem.fixed && q.cap > NGI_SHQ && rec * q.waves * q.cap > *mem.bytes) q.cap >>= 1;
@@ -315,7 +325,7 @@ static int launch_pk(const RenderArgs& a, unsigned long long* next, LaneMem mem,
         if ((s = mem.reserve(rec * q.waves * q.cap))) return s;
         q.rec = reinterpret_cast<float4*>(*mem.ptr);
     }
-    kern<<<grid, NGI_MK_BLOCK, lds, st>>>(a, next, q);
+    kern<<<grid, NGI_MK_BLOCK, lds, st>>>(b, next, q);
     NGI_HIP_CHECK(hipGetLastError());
     return NGI_OK;
 }
@@ -538,7 +548,8 @@ RenderArgs Session::args(void* target_film) const {
     // 36-triangle Cornell box: +27% / +40% with chunks of 128); on large ones
     // exact refills keep each wavefront's paths spread over the frontier
     // (chunks cost 5-10% on the 77k-triangle nave and the sphere field).
-    a.path_chunk = scene->dev->view.num_tris < NGI_CHUNKED_FEED_TRIS ? 128u : 0u;
+    a.path_chunk = scene->dev->view.num_tris < NGI_CHUNKED_FEED_TRIS ? 128u : 0u;   // persistent_feed limits it
+    a.path_lanes = 64;
     return a;
 }
 

@@ -434,3 +434,23 @@ def test_full_size_sphere_field_fp32_against_fp64_shading():
         out[prec], st = ngi.render(s, p)
         assert st["samples"] == 1024 * 1024 * 4 and st["shadow_rays"] > 0
     _crn_close(out[ngi.PRECISION_FP32_FP64ACC], out[ngi.PRECISION_FP64_ALL], 2e-4, frac=0.97, mean_rtol=1e-3)
+
+
+@pytest.mark.parametrize("kind", [ngi.GEN_BATCH_ROOM, ngi.GEN_NAVE])
+@pytest.mark.parametrize("renderer", ["pt", "ptdirect", "ltdirect"])
+@pytest.mark.parametrize("w,h", [(1, 1), (33, 1), (257, 16), (640, 256), (641, 256)])
+def test_launches_smaller_than_the_device_equal_one_block(kind, renderer, w, h):
+    """How a small launch spreads its paths over wavefronts (32 or 64 lanes
+    each, chunk sizes) changes only which lane runs a path: the film equals
+    that of a single block fed 64 lanes at a time but for the order of the
+    FP64 additions."""
+    s = ngi.Scene.generate(kind, 3, w / h, 400)
+    p = _params(renderer, w, h, 1, 7, rr_depth=3, engine=ngi.ENGINE_PERSISTENT)
+    p.num_samples = w * h
+    one = _params(renderer, w, h, 1, 7, rr_depth=3, engine=ngi.ENGINE_PERSISTENT)
+    one.num_samples = w * h
+    one.paths_in_flight = 1
+    (g, st), (o, so) = ngi.render(s, p), ngi.render(s, one)
+    assert st["samples"] == so["samples"] == w * h
+    assert st["extension_rays"] == so["extension_rays"] and st["shadow_rays"] == so["shadow_rays"]
+    assert np.abs(g - o).max() <= 1e-9 * max(1.0, np.abs(o).max())
