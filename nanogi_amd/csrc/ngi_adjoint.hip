@@ -33,9 +33,9 @@
 //
 // Layout: the persistent engine's regenerating lanes; per-lane vertex
 // records (prim, P_j) in HBM as [record][lane] float4; per-block FP64 LDS
-// accumulators for the first NGI_ADJ_LDS_PRIMS primitives, flushed with one
-// FP64 global atomic per value and block; the rest go straight to global
-// FP64 atomics.
+// accumulators (NGI_ADJ_LDS_PRIMS, NGI_ADJ_LDS_LIGHTS), flushed with one FP64
+// global atomic per value and block; the rest go straight to global FP64
+// atomics.
 #include <algorithm>
 #include <chrono>
 #include <cstring>
@@ -46,16 +46,35 @@
 namespace ngi {
 
 #define NGI_ADJ_BLOCK 256
-// Ended paths are replaced at once: waiting for 16 of them, as the forward
-// persistent kernels do, made the 64-spp replay on the nave 35.83 ms against
-// 34.58 ms.
-// Minimum waves per SIMD for the adjoint kernel's register allocation: 4
-// (128 VGPRs) measured fastest on the nave (38.2 ms per 64-spp replay against
-// 44.8 ms unconstrained at 140 VGPRs / 3 waves, 38.6 ms at 5 waves).
+// Minimum waves per SIMD for the register allocation of the kernel that runs
+// every traversal to its end: 4 (128 VGPRs) measured fastest on the nave (38.2
+// ms per 64-spp replay against 44.8 ms unconstrained at 140 VGPRs / 3 waves,
+// 38.6 ms at 5 waves).
 #ifndef NGI_ADJ_WAVES
 #define NGI_ADJ_WAVES 4
 #endif
+// The resumable kernel at 5 waves (96 VGPRs): 8.4M paths on the nave 12.2 ms
+// against 12.9 ms at 4.
+#ifndef NGI_ADJ_RESUME_WAVES
+#define NGI_ADJ_RESUME_WAVES 5
+#endif
+// The sums of ended paths wait in their lanes until NGI_ADJ_FINISH of them are
+// finished together; 4.2M paths of 8 / 16 / 24: nave 6.77 / 6.68 / 6.91 ms,
+// 8k-triangle room 4.12 / 4.08 / 4.07.  Without chunks new paths start 16 at a
+// time (one atomic on the launch's counter each time, as the forward kernels).
+#ifndef NGI_ADJ_FINISH
+#define NGI_ADJ_FINISH 16
+#endif
+#ifndef NGI_ADJ_PATH_REFILL
+#define NGI_ADJ_PATH_REFILL 16
+#endif
+// Gradients accumulated per block in LDS: those of the first
+// NGI_ADJ_LDS_PRIMS primitives (a power of two) that its paths meet, and of the
+// first NGI_ADJ_LDS_LIGHTS lights.  An emitter or a floor without a slot is one
+// address in HBM for every path's FP64 atomics: 4.2M ptdirect paths on a sphere
+// field, whose emitter is its last primitive, took 59 ms, now 2.8.
 #define NGI_ADJ_LDS_PRIMS 256
+#define NGI_ADJ_LDS_LIGHTS 256
 
 // Zero-parameter mask per primitive: bits 0-2 reflectance channel is 0,
 // bits 3-5 radiance channel is 0 (the replay tables hold 1 there).
@@ -77,10 +96,11 @@ struct AdjArgs {
     int nprims;
 };
 
-__device__ __forceinline__ void grad_add(double* lds, double* glob, int nlds, int prim, int c, float v) {
+// Adds to channel c of a gradient: its slot in LDS, if it has one, or in HBM.
+__device__ __forceinline__ void grad_add(double* lds, double* glob, bool in_lds, int c, float v) {
     if (v == 0.0f) return;
-    if (prim < nlds) atomicAdd(lds + 3 * prim + c, (double)v);
-    else unsafeAtomicAdd(glob + 3 * prim + c, (double)v);
+    if (in_lds) atomicAdd(lds + c, (double)v);
+    else unsafeAtomicAdd(glob + c, (double)v);
 }
 
 // Adjoint sums of one path: SA / SB = weighted contributions with no / one
@@ -94,8 +114,9 @@ struct AdjPath {
 
 // A contribution C at pixel `pix` from emitter primitive `emitter_prim`.
 template <bool ZEROS>
-__device__ __forceinline__ void adj_contribute(const AdjArgs& g, const DevPrim<float>* prims, double* sL, int nlds, AdjPath& q, int pix,
-                                               f3 C, int emitter_prim) {
+__device__ __forceinline__ void adj_contribute(const AdjArgs& g, const DevPrim<float>* prims, const DevLight<float>* lights, double* sL,
+                                               AdjPath& q, int pix, f3 C, int light) {
+    const int emitter_prim = lights[light].prim;
     const float* gp = g.dLdI + 3 * (size_t)pix;
     const float gC[3] = {gp[0] * C.x * g.scale, gp[1] * C.y * g.scale, gp[2] * C.z * g.scale};
     const DevPrim<float>& E = prims[emitter_prim];
@@ -106,7 +127,7 @@ __device__ __forceinline__ void adj_contribute(const AdjArgs& g, const DevPrim<f
         const uint32_t z = (q.zc >> (2 * c)) & 3u;
         const bool le_zero = (zm & (NGI_ADJ_LEZERO << c)) != 0;
         if (z == 0) {
-            grad_add(sL, g.gLe, nlds, emitter_prim, c, gC[c] / E.Le[c]);   // Le~ = 1 where Le = 0
+            grad_add(sL + 3 * light, g.gLe + 3 * (size_t)emitter_prim, light < NGI_ADJ_LDS_LIGHTS, c, gC[c] / E.Le[c]);   // Le~ = 1 where Le = 0
             if (!le_zero) sa[c] += gC[c];
         } else if (z == 1 && !le_zero) {
             sb[c] += gC[c];
@@ -132,30 +153,76 @@ __device__ __forceinline__ void adj_record(const AdjArgs& g, uint32_t gid, AdjPa
     q.nrec++;
 }
 
-// End of a path: the reflectance gradients of its records.
+// The LDS slot of a primitive's reflectance gradient: the slots of a block go
+// to the first primitives that ask for them (`tags`: the owners, -1 free;
+// without tags where every primitive has a slot), so that the surfaces which
+// most paths meet have one whatever their numbers.  -1: none.
+__device__ __forceinline__ int reflectance_slot(const AdjArgs& g, int* tags, int prim) {
+    if (g.nprims <= NGI_ADJ_LDS_PRIMS) return prim;
+    const int s = prim & (NGI_ADJ_LDS_PRIMS - 1);
+    int t = __hip_atomic_load(tags + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (t == -1) {
+        t = atomicCAS(tags + s, -1, prim);
+        if (t == -1) t = prim;
+    }
+    return t == prim ? s : -1;
+}
+
+// The reflectance gradient of one record of a path whose sums are sa, sb.
 template <bool ZEROS>
-__device__ __forceinline__ void adj_finish(const AdjArgs& g, const DevPrim<float>* prims, double* sR, int nlds, uint32_t gid, const AdjPath& q) {
-    const float sa[3] = {q.SA.x, q.SA.y, q.SA.z}, sb[3] = {q.SB.x, q.SB.y, q.SB.z};
-    for (int r = 0; r < q.nrec; ++r) {
-        const float4 e = g.rec[(size_t)r * g.lanes + gid];
-        const uint32_t w = __float_as_uint(e.w);
-        const int m = (int)(w & NGI_ADJ_PRIM_MASK);
-        const DevPrim<float>& P = prims[m];
-        const uint32_t zm = ZEROS ? g.zmask[m] : 0u;
-        const float pa[3] = {e.x, e.y, e.z};
+__device__ __forceinline__ void adj_record_sums(const AdjArgs& g, const DevPrim<float>* prims, double* sR, int* tags, float4 e,
+                                                const float sa[3], const float sb[3]) {
+    const uint32_t w = __float_as_uint(e.w);
+    const int m = (int)(w & NGI_ADJ_PRIM_MASK);
+    const DevPrim<float>& P = prims[m];
+    const uint32_t zm = ZEROS ? g.zmask[m] : 0u;
+    const float pa[3] = {e.x, e.y, e.z};
+    const int slot = reflectance_slot(g, tags, m);
+    double* lds = sR + 3 * (slot < 0 ? 0 : slot);
+    double* glob = g.gR + 3 * (size_t)m;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            if (!(zm & (NGI_ADJ_RZERO << c))) grad_add(sR, g.gR, nlds, m, c, (sa[c] - pa[c]) / P.R[c]);
-            else if (w & (1u << (29 + c))) grad_add(sR, g.gR, nlds, m, c, sb[c]);
-        }
+    for (int c = 0; c < 3; ++c) {
+        if (!(zm & (NGI_ADJ_RZERO << c))) grad_add(lds, glob, slot >= 0, c, (sa[c] - pa[c]) / P.R[c]);
+        else if (w & (1u << (29 + c))) grad_add(lds, glob, slot >= 0, c, sb[c]);
     }
 }
 
+// End of a path: the reflectance gradients of its records.
+template <bool ZEROS>
+__device__ __forceinline__ void adj_finish(const AdjArgs& g, const DevPrim<float>* prims, double* sR, int* tags, uint32_t gid, const AdjPath& q) {
+    const float sa[3] = {q.SA.x, q.SA.y, q.SA.z}, sb[3] = {q.SB.x, q.SB.y, q.SB.z};
+    for (int r = 0; r < q.nrec; ++r) adj_record_sums<ZEROS>(g, prims, sR, tags, g.rec[(size_t)r * g.lanes + gid], sa, sb);
+}
+
+// adj_finish for all lanes set in `fin` at once (every lane of the wavefront
+// calls this): the lanes share out the records of the ended paths.
+template <bool ZEROS>
+__device__ __forceinline__ void adj_finish_wave(const AdjArgs& g, const DevPrim<float>* prims, double* sR, int* tags, uint32_t gid, const AdjPath& q,
+                                                unsigned long long fin) {
+    const uint32_t lane = __lane_id();
+    const uint32_t n = (uint32_t)__popcll(fin), step = 64u / n;   // lanes per path
+    // Lane j: path number j % n of the set, records j / n, j / n + step, ...
+    const uint32_t first = lane / n, which = lane % n;
+    const uint32_t rank = (uint32_t)__popcll(fin & ((1ull << lane) - 1ull));
+    const bool mine = (fin >> lane) & 1ull;
+    // The lanes of the set, compacted: the others send to the lanes behind.
+    const uint32_t slot = mine ? rank : n + (lane - rank);
+    const int owner = __shfl(__builtin_amdgcn_ds_permute((int)(slot << 2), (int)lane), (int)which);
+    const float sa[3] = {__shfl(q.SA.x, owner), __shfl(q.SA.y, owner), __shfl(q.SA.z, owner)};
+    float sb[3] = {0.0f, 0.0f, 0.0f};
+    if (ZEROS) sb[0] = __shfl(q.SB.x, owner), sb[1] = __shfl(q.SB.y, owner), sb[2] = __shfl(q.SB.z, owner);
+    const int owner_rec = __shfl(q.nrec, owner);
+    const uint32_t nrec = first < step ? (uint32_t)owner_rec : 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // other lanes' records
+    for (uint32_t r = first; r < nrec; r += step) adj_record_sums<ZEROS>(g, prims, sR, tags, g.rec[(size_t)r * g.lanes + (gid - lane) + owner], sa, sb);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // The light picked by a NEE sample (the draw of sample_light).
-__device__ __forceinline__ int nee_light(const DevScene& sc, const DevLight<float>* lights, U4 rn) {
+__device__ __forceinline__ int nee_light(const DevScene& sc, U4 rn) {
     int li = (int)(u24f(rn.x) * (float)sc.num_lights);
     li = li < 0 ? 0 : (li > sc.num_lights - 1 ? sc.num_lights - 1 : li);
-    return lights[li].prim;
+    return li;
 }
 
 // ZEROS: some parameter channel is zero (the zero bookkeeping is compiled in
@@ -163,11 +230,14 @@ __device__ __forceinline__ int nee_light(const DevScene& sc, const DevLight<floa
 template <bool DIRECT, int WIDTH, bool ZEROS>
 __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_kernel(RenderArgs a, AdjArgs g, unsigned long long* next) {
     extern __shared__ double adj_smem[];
-    const int nlds = min(g.nprims, NGI_ADJ_LDS_PRIMS);
+    const int nR = 3 * min(g.nprims, NGI_ADJ_LDS_PRIMS), nL = 3 * min(a.sc.num_lights, NGI_ADJ_LDS_LIGHTS);
     double* sR = adj_smem;
-    double* sL = adj_smem + 3 * nlds;
-    uint32_t* stk = reinterpret_cast<uint32_t*>(adj_smem + 6 * nlds);
-    for (int i = threadIdx.x; i < 6 * nlds; i += NGI_ADJ_BLOCK) adj_smem[i] = 0.0;
+    double* sL = adj_smem + nR;
+    const int ntags = g.nprims > NGI_ADJ_LDS_PRIMS ? NGI_ADJ_LDS_PRIMS : 0;
+    int* tags = reinterpret_cast<int*>(adj_smem + nR + nL);
+    uint32_t* stk = reinterpret_cast<uint32_t*>(tags + ntags);
+    for (int i = threadIdx.x; i < nR + nL; i += NGI_ADJ_BLOCK) adj_smem[i] = 0.0;
+    for (int i = threadIdx.x; i < ntags; i += NGI_ADJ_BLOCK) tags[i] = -1;
     __syncthreads();
 
     const DevScene& sc = a.sc;
@@ -231,7 +301,7 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_kernel(R
                 TraceHit sh;
                 TraceCounters tc{0, 0};
                 if (!trace<WIDTH, true, false>(sc, sr, sh, tc, my_stk, NGI_ADJ_BLOCK))
-                    adj_contribute<ZEROS>(g, prims, sL, nlds, q, target, C, nee_light(sc, lights, rn));
+                    adj_contribute<ZEROS>(g, prims, lights, sL, q, target, C, nee_light(sc, rn));
             }
         }
         f3 wo(0.0f);
@@ -255,7 +325,7 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_kernel(R
                     if (!DIRECT && (htype & NGI_PRIM_L)) {
                         const DevPrim<float>& hm = prims[hp];
                         if (hm.light >= 0 && lights[hm.light].type == NGI_LIGHT_AREA && dot(ns.n, -wo) > 0.0f)
-                            adj_contribute<ZEROS>(g, prims, sL, nlds, q, pixel, T * f3(hm.Le[0], hm.Le[1], hm.Le[2]), hp);
+                            adj_contribute<ZEROS>(g, prims, lights, sL, q, pixel, T * f3(hm.Le[0], hm.Le[1], hm.Le[2]), hm.light);
                     }
                     if (a.rr_depth >= 0 && nv >= a.rr_depth) {
                         if (u24f(rx.w) > a.rr_prob_f) alive = false;
@@ -271,37 +341,57 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_kernel(R
             }
         }
         if (!alive) {
-            adj_finish<ZEROS>(g, prims, sR, nlds, gid, q);
+            adj_finish<ZEROS>(g, prims, sR, tags, gid, q);
             active = false;
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 3 * nlds; i += NGI_ADJ_BLOCK) {
-        if (sR[i] != 0.0) unsafeAtomicAdd(g.gR + i, sR[i]);
-        if (sL[i] != 0.0) unsafeAtomicAdd(g.gLe + i, sL[i]);
-    }
+    for (int i = threadIdx.x; i < nR; i += NGI_ADJ_BLOCK)
+        if (sR[i] != 0.0) unsafeAtomicAdd(g.gR + (ntags ? 3 * (size_t)tags[i / 3] + i % 3 : (size_t)i), sR[i]);
+    for (int i = threadIdx.x; i < nL; i += NGI_ADJ_BLOCK)
+        if (sL[i] != 0.0) unsafeAtomicAdd(g.gLe + 3 * (size_t)lights[i / 3].prim + i % 3, sL[i]);
 }
 
-// The adjoint kernel with resumable extension traversals (wide BVH): a
-// wavefront stops traversing once at most NGI_ADJ_KEEP of its lanes are still
-// inside the tree; the others complete their vertices and start their next
-// rays while those wait, their traversal state, direction and roulette number
-// parked in LDS.  NEE shadow rays are traced where they are made (their
-// contributions enter the adjoint sums before the next vertex record), on a
-// second LDS stack.  Every path takes the same vertices as in adjoint_kernel.
+// The adjoint kernel with resumable traversals (wide BVH): a wavefront stops
+// traversing once a few of its lanes are still inside the tree; the others
+// complete their vertices and start their next rays while those wait, their
+// traversal state, direction and roulette number parked in LDS.  A lane's
+// NEE shadow ray runs in the same loop before its extension ray (their
+// contributions enter the adjoint sums before the next vertex record): traced
+// where it was made, it kept few lanes busy for its longest ray.  Records of
+// ended paths are shared out over the wavefront's lanes.  Every path takes the
+// same vertices as in adjoint_kernel.
+//
+// Bound by the traversals, as the forward kernel (8.4M ptdirect paths on the
+// nave: forward 10.5 ms).  Measured there: shadow rays in place, each path
+// finished by its own lane, one counter atomic per refill 15.0 ms; shadow rays
+// in the loop 15.0; with paths finished 16 at a time 13.1 (without the former
+// 14.9); 16 lanes left waiting instead of 8 12.9; 5 waves per SIMD 12.2.  4.2M
+// paths per call with chunks of path ids: Cornell box pt 3.7 -> 1.8 ms,
+// ptdirect 3.9 -> 3.1.  8 / 16 lanes waiting: sphere field (glossy) pt 1.59 /
+// 1.78 ms, 8k-triangle room ptdirect 4.28 / 4.08, nave 6.78 / 6.68.
 #ifndef NGI_ADJ_KEEP
 #define NGI_ADJ_KEEP 8
 #endif
+#ifndef NGI_ADJ_KEEP_DIFFUSE
+#define NGI_ADJ_KEEP_DIFFUSE 16
+#endif
+// Parked words of ptdirect behind the extension ray's: direction of the
+// vertex's shadow ray, its contribution, pixel and emitter primitive.
+enum { APK_SX = PK_WORDS, APK_SY, APK_SZ, APK_CX, APK_CY, APK_CZ, APK_PIXEL, APK_EMITTER, APK_WORDS };
 template <bool DIRECT, bool ZEROS>
-__global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_resume_kernel(RenderArgs a, AdjArgs g, unsigned long long* next) {
-    // LDS: the FP64 accumulators, then extension stacks, shadow stacks
-    // (a.sc.stack_entries words per lane each) and the parked lane state.
+__global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_RESUME_WAVES) adjoint_resume_kernel(RenderArgs a, AdjArgs g, unsigned long long* next) {
+    // LDS: the FP64 accumulators, then the traversal stacks
+    // (a.sc.stack_entries words per lane) and the parked lane state.
     extern __shared__ double adj_smem[];
-    const int nlds = min(g.nprims, NGI_ADJ_LDS_PRIMS);
+    const int nR = 3 * min(g.nprims, NGI_ADJ_LDS_PRIMS), nL = 3 * min(a.sc.num_lights, NGI_ADJ_LDS_LIGHTS);
     double* sR = adj_smem;
-    double* sL = adj_smem + 3 * nlds;
-    uint32_t* words = reinterpret_cast<uint32_t*>(adj_smem + 6 * nlds);
-    for (int i = threadIdx.x; i < 6 * nlds; i += NGI_ADJ_BLOCK) adj_smem[i] = 0.0;
+    double* sL = adj_smem + nR;
+    const int ntags = g.nprims > NGI_ADJ_LDS_PRIMS ? NGI_ADJ_LDS_PRIMS : 0;
+    int* tags = reinterpret_cast<int*>(adj_smem + nR + nL);
+    uint32_t* words = reinterpret_cast<uint32_t*>(tags + ntags);
+    for (int i = threadIdx.x; i < nR + nL; i += NGI_ADJ_BLOCK) adj_smem[i] = 0.0;
+    for (int i = threadIdx.x; i < ntags; i += NGI_ADJ_BLOCK) tags[i] = -1;
     __syncthreads();
 
     const DevScene& sc = a.sc;
@@ -311,9 +401,8 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_resume_k
     const int max_nv = (a.max_nv < 0 || a.max_nv > NGI_MAX_VERTICES) ? NGI_MAX_VERTICES : a.max_nv;
     const uint32_t lane = __lane_id();
     const uint32_t gid = blockIdx.x * NGI_ADJ_BLOCK + threadIdx.x;
-    uint32_t* ext_stk = words + threadIdx.x;
-    uint32_t* sh_stk = words + (size_t)sc.stack_entries * NGI_ADJ_BLOCK + threadIdx.x;
-    uint32_t* pk = words + (size_t)2 * sc.stack_entries * NGI_ADJ_BLOCK + threadIdx.x;
+    uint32_t* lds_stk = words + threadIdx.x;
+    uint32_t* pk = words + (size_t)sc.stack_entries * NGI_ADJ_BLOCK + threadIdx.x;
     const bool geometry = sc.num_tris != 0;
 
     f3 T(0.0f), wi(0.0f);
@@ -322,12 +411,33 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_resume_k
     int type = 0, prim = 0, nv = 0, pixel = 0;
     uint32_t c0 = 0, c1 = 0;
     bool active = false;      // the lane holds a path
-    bool busy = false;        // ... whose extension ray is being traced
-    bool exhausted = false;   // wave-uniform: no path ids left
+    bool busy = false;        // ... one of whose rays is being traced
+    bool shadow = false;      // ... the vertex's shadow ray, not its extension ray
+    bool extends = false;     // the path goes on after its shadow ray
+    bool ended = false;       // the lane holds the sums of a path that has ended
+    PathFeed feed;
     for (;;) {
-        // Vertices whose extension rays have finished (hit, emission for pt,
-        // Russian roulette).
-        if (active && !busy) {
+        // Lanes whose shadow rays have finished contribute and start the
+        // vertex's extension ray, or end their paths.
+        if (DIRECT && active && !busy && shadow) {
+            if (parked_hit<NGI_ADJ_BLOCK>(pk).leaf < 0) {
+                const f3 C = f3(__uint_as_float(pk[APK_CX * NGI_ADJ_BLOCK]), __uint_as_float(pk[APK_CY * NGI_ADJ_BLOCK]),
+                                __uint_as_float(pk[APK_CZ * NGI_ADJ_BLOCK]));
+                adj_contribute<ZEROS>(g, prims, lights, sL, q, (int)pk[APK_PIXEL * NGI_ADJ_BLOCK], C, (int)pk[APK_EMITTER * NGI_ADJ_BLOCK]);
+            }
+            shadow = false;
+            if (extends) {
+                Trav8 tv;
+                trav8_begin(FLT_MAX, tv);
+                park_trav<NGI_ADJ_BLOCK>(pk, tv);
+                busy = true;
+            } else {
+                ended = true;
+                active = false;
+            }
+        } else if (active && !busy) {
+            // Vertices whose extension rays have finished (hit, emission for
+            // pt, Russian roulette).
             const TraceHit h = parked_hit<NGI_ADJ_BLOCK>(pk);
             bool alive = h.leaf >= 0;
             if (alive) {
@@ -337,7 +447,7 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_resume_k
                 if (!DIRECT && (htype & NGI_PRIM_L)) {
                     const DevPrim<float>& hm = prims[hp];
                     if (hm.light >= 0 && lights[hm.light].type == NGI_LIGHT_AREA && dot(ns.n, -wo) > 0.0f)
-                        adj_contribute<ZEROS>(g, prims, sL, nlds, q, pixel, T * f3(hm.Le[0], hm.Le[1], hm.Le[2]), hp);
+                        adj_contribute<ZEROS>(g, prims, lights, sL, q, pixel, T * f3(hm.Le[0], hm.Le[1], hm.Le[2]), hm.light);
                 }
                 if (a.rr_depth >= 0 && nv >= a.rr_depth) {
                     if (parked_urr<NGI_ADJ_BLOCK>(pk) > a.rr_prob_f) alive = false;
@@ -351,37 +461,36 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_resume_k
                 nv++;
             }
             if (!alive) {
-                adj_finish<ZEROS>(g, prims, sR, nlds, gid, q);
+                ended = true;
                 active = false;
             }
         }
-        if (!exhausted) {
-            const unsigned long long need = __ballot(!active);
-            if (need) {
-                const int leader = __ffsll((long long)need) - 1;
-                unsigned long long base = 0;
-                if ((int)lane == leader) base = atomicAdd(next, (unsigned long long)__popcll(need));
-                base = __shfl(base, leader);
-                if (base + __popcll(need) >= a.path_count) exhausted = true;
-                if (!active) {
-                    const unsigned long long local = base + (unsigned long long)__popcll(need & ((1ull << lane) - 1ull));
-                    if (local < a.path_count) {
-                        path_coords(a, a.path_begin + local, c0, c1, pixel);
-                        T = f3(1.0f);
-                        type = NGI_PRIM_E;
-                        prim = sc.sensor_prim;
-                        s.p = cam.eye;
-                        s.degenerate = true;
-                        wi = f3(0.0f);
-                        nv = 1;
-                        q = AdjPath{f3(0.0f), f3(0.0f), 0u, 0};
-                        active = true;
-                    }
+        const unsigned long long fin = __ballot(ended);
+        if (fin && (__popcll(fin) >= NGI_ADJ_FINISH || __ballot(active) == 0)) {
+            adj_finish_wave<ZEROS>(g, prims, sR, tags, gid, q, fin);
+            ended = false;
+        }
+        if (!feed.done()) {
+            const unsigned long long need = __ballot(!active && !ended);
+            if (need && (a.path_chunk || __popcll(need) >= NGI_ADJ_PATH_REFILL || __ballot(active || ended) == 0)) {
+                const unsigned long long id = feed.take<true>(next, a.path_count, need, a.path_chunk);
+                if (id != ~0ull) {
+                    path_coords(a, a.path_begin + id, c0, c1, pixel);
+                    T = f3(1.0f);
+                    type = NGI_PRIM_E;
+                    prim = sc.sensor_prim;
+                    s.p = cam.eye;
+                    s.degenerate = true;
+                    wi = f3(0.0f);
+                    nv = 1;
+                    q = AdjPath{f3(0.0f), f3(0.0f), 0u, 0};
+                    active = true;
                 }
             }
         }
         // Next vertex of every path not inside the tree: record, NEE,
-        // direction sample, extension ray.
+        // direction sample, then the shadow ray or, without one, the
+        // extension ray.
         if (active && !busy) {
             bool alive = nv < max_nv;
             if (alive && (type & (NGI_PRIM_D | NGI_PRIM_G)) && q.nrec < g.max_rec) adj_record<ZEROS>(g, gid, q, prim);
@@ -390,11 +499,22 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_resume_k
                 TraceRay sr;
                 int target;
                 const f3 C = nee_contribution<float>(sc, cam, prims, type, prim, s, wi, T, rn, a.w, a.h, pixel, sr, target);
-                if (!is_zero(C)) {
-                    TraceHit sh;
-                    TraceCounters tc{0, 0};
-                    if (!trace<8, true, false>(sc, sr, sh, tc, sh_stk, NGI_ADJ_BLOCK))
-                        adj_contribute<ZEROS>(g, prims, sL, nlds, q, target, C, nee_light(sc, lights, rn));
+                const int emitter = nee_light(sc, rn);
+                if (!is_zero(C) && !geometry) {
+                    adj_contribute<ZEROS>(g, prims, lights, sL, q, target, C, emitter);
+                } else if (!is_zero(C)) {
+                    Trav8 tv;
+                    trav8_begin(sr.tmax, tv);
+                    park_trav<NGI_ADJ_BLOCK>(pk, tv);
+                    pk[APK_SX * NGI_ADJ_BLOCK] = __float_as_uint(sr.dx);
+                    pk[APK_SY * NGI_ADJ_BLOCK] = __float_as_uint(sr.dy);
+                    pk[APK_SZ * NGI_ADJ_BLOCK] = __float_as_uint(sr.dz);
+                    pk[APK_CX * NGI_ADJ_BLOCK] = __float_as_uint(C.x);
+                    pk[APK_CY * NGI_ADJ_BLOCK] = __float_as_uint(C.y);
+                    pk[APK_CZ * NGI_ADJ_BLOCK] = __float_as_uint(C.z);
+                    pk[APK_PIXEL * NGI_ADJ_BLOCK] = (uint32_t)target;
+                    pk[APK_EMITTER * NGI_ADJ_BLOCK] = (uint32_t)emitter;
+                    shadow = busy = true;
                 }
             }
             if (alive) {
@@ -408,15 +528,18 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_resume_k
                     if (alive) T = T * wgt;
                 }
                 if (alive) {
-                    Trav8 tv;
-                    trav8_begin(FLT_MAX, tv);
-                    park_trav<NGI_ADJ_BLOCK>(pk, tv);
                     park_dir<NGI_ADJ_BLOCK>(pk, wo, u24f(rx.w));
-                    busy = geometry;
+                    if (!shadow) {
+                        Trav8 tv;
+                        trav8_begin(FLT_MAX, tv);
+                        park_trav<NGI_ADJ_BLOCK>(pk, tv);
+                        busy = geometry;
+                    }
                 }
             }
-            if (!alive) {
-                adj_finish<ZEROS>(g, prims, sR, nlds, gid, q);
+            extends = alive;
+            if (!alive && !shadow) {
+                ended = true;
                 active = false;
             }
         }
@@ -426,25 +549,25 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_resume_k
         s.degenerate = false;
         type = prim = 0;
         if (__ballot(active) == 0) {
-            if (exhausted) break;
+            if (feed.done() && __ballot(ended) == 0) break;
             continue;
         }
         if (__ballot(busy)) {
             // Lanes without a ray load and store back what they parked last.
             Trav8 tv = parked_trav<NGI_ADJ_BLOCK>(pk);
-            const f3 d = parked_dir<NGI_ADJ_BLOCK>(pk);
+            const f3 d = parked_dir<NGI_ADJ_BLOCK>(pk + (DIRECT && shadow ? (APK_SX - PK_WX) * NGI_ADJ_BLOCK : 0));
             const RayPre r = make_pre(TraceRay{s.p.x, s.p.y, s.p.z, d.x, d.y, d.z, NGI_EPS_F, FLT_MAX});
-            const int keep = __builtin_amdgcn_readfirstlane(exhausted ? 0 : NGI_ADJ_KEEP);
+            const int keep = __builtin_amdgcn_readfirstlane(feed.done() ? (int)__popcll(__ballot(busy)) / 4 : (a.sc.any_glossy ? NGI_ADJ_KEEP : NGI_ADJ_KEEP_DIFFUSE));
             TraceCounters tc{0, 0};
-            trav8_run<false>(sc, r, NGI_EPS_F, tv, busy, keep, tc, ext_stk, NGI_ADJ_BLOCK);
+            trav8_run<false, DIRECT>(sc, r, NGI_EPS_F, tv, busy, keep, tc, lds_stk, NGI_ADJ_BLOCK, shadow);
             park_trav<NGI_ADJ_BLOCK>(pk, tv);
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 3 * nlds; i += NGI_ADJ_BLOCK) {
-        if (sR[i] != 0.0) unsafeAtomicAdd(g.gR + i, sR[i]);
-        if (sL[i] != 0.0) unsafeAtomicAdd(g.gLe + i, sL[i]);
-    }
+    for (int i = threadIdx.x; i < nR; i += NGI_ADJ_BLOCK)
+        if (sR[i] != 0.0) unsafeAtomicAdd(g.gR + (ntags ? 3 * (size_t)tags[i / 3] + i % 3 : (size_t)i), sR[i]);
+    for (int i = threadIdx.x; i < nL; i += NGI_ADJ_BLOCK)
+        if (sL[i] != 0.0) unsafeAtomicAdd(g.gLe + 3 * (size_t)lights[i / 3].prim + i % 3, sL[i]);
 }
 
 template <bool DIRECT, int WIDTH, bool ZEROS, bool RESUME>
@@ -511,12 +634,13 @@ int render_adjoint(ngi_scene* scene, const ngi_render_params& p, const double* d
     const int nprims = (int)scene->prims.size();
     const bool direct = p.renderer == NGI_RENDERER_PTDIRECT;
     const int width = scene->dev->view.bvh_width;
-    const int nlds = std::min(nprims, NGI_ADJ_LDS_PRIMS);
-    // Resumable traversals (wide BVH) while their LDS leaves the kernel its
-    // occupancy of NGI_ADJ_WAVES blocks per CU.
-    const size_t resume_lds = (size_t)6 * nlds * 8 + ((size_t)2 * scene->dev->view.stack_entries + PK_WORDS) * NGI_ADJ_BLOCK * 4;
-    const bool resume = width == 8 && resume_lds * NGI_ADJ_WAVES <= NGI_CU_LDS_BYTES;
-    const size_t lds = resume ? resume_lds : (size_t)6 * nlds * 8 + (width == 8 ? (size_t)scene->dev->view.stack_entries * NGI_ADJ_BLOCK * 4 : 0);
+    const size_t sums = (size_t)24 * (std::min(nprims, NGI_ADJ_LDS_PRIMS) + std::min(scene->dev->view.num_lights, NGI_ADJ_LDS_LIGHTS)) +
+                        (nprims > NGI_ADJ_LDS_PRIMS ? 4 * NGI_ADJ_LDS_PRIMS : 0);
+    // Resumable traversals (wide BVH) while their LDS leaves the kernel
+    // NGI_RESUME_MIN_BLOCKS blocks per CU, as the forward kernels.
+    const size_t resume_lds = sums + ((size_t)scene->dev->view.stack_entries + (direct ? APK_WORDS : PK_WORDS)) * NGI_ADJ_BLOCK * 4;
+    const bool resume = width == 8 && resume_lds * NGI_RESUME_MIN_BLOCKS <= NGI_CU_LDS_BYTES;
+    const size_t lds = resume ? resume_lds : sums + (width == 8 ? (size_t)scene->dev->view.stack_entries * NGI_ADJ_BLOCK * 4 : 0);
     unsigned grid = 1;
     std::vector<void*> mem;
     auto cleanup = [&]() {
@@ -566,6 +690,9 @@ int render_adjoint(ngi_scene* scene, const ngi_render_params& p, const double* d
         cleanup();
         return st;
     }
+    grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(grid, (total + NGI_ADJ_BLOCK - 1) / NGI_ADJ_BLOCK));
+    a.path_count = total;
+    persistent_feed(a, NGI_ADJ_BLOCK, 0, false, &grid);
     g.lanes = grid * NGI_ADJ_BLOCK;
     void *d_dl = nullptr, *d_rec = nullptr, *d_gR = nullptr, *d_gL = nullptr, *d_next = nullptr;
     void *d_rp = nullptr, *d_rl = nullptr, *d_zm = nullptr;
@@ -605,7 +732,6 @@ int render_adjoint(ngi_scene* scene, const ngi_render_params& p, const double* d
     a.sc.prims_f = reinterpret_cast<const DevPrim<float>*>(d_rp);
     a.sc.lights_f = reinterpret_cast<const DevLight<float>*>(d_rl);
     a.path_begin = 0;
-    a.path_count = total;
     a.sample_base = 0;
     if (!st && total) {
         unsigned long long* nx = reinterpret_cast<unsigned long long*>(d_next);

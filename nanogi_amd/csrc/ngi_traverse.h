@@ -401,9 +401,11 @@ __device__ __forceinline__ void trav8_begin(float tmax, Trav8& t) {
 // 8.43 -> 7.96, 7.4M with FP64 shading 4.95 -> 4.39, ltdirect on the nave
 // 10.20 -> 9.27, adjoint replay 15.6 -> 14.9.  (Fetching the next children
 // too before a leaf's second triangle needs 24 registers more: 8.88.)
-template <bool COUNT>
+// With MIXED, the lanes with `any` set stop at their first hit (t.h.leaf tells
+// whether there is one).
+template <bool COUNT, bool MIXED = false>
 __device__ __forceinline__ void trav8_run(const DevScene& sc, const RayPre& r, float tmin, Trav8& t, bool& busy, int keep,
-                                          TraceCounters& cnt, uint32_t* lds_stack, int lane_stride) {
+                                          TraceCounters& cnt, uint32_t* lds_stack, int lane_stride, bool any = false) {
     int32_t ref = 0;
     if (busy && t.mask != NGI_TRAV8_FRESH) ref = next_child(sc, r, t.cur, t.mask);
     do {
@@ -430,7 +432,10 @@ __device__ __forceinline__ void trav8_run(const DevScene& sc, const RayPre& r, f
             }
             if (more) ref = next_child(sc, r, t.cur, t.mask);
         }
-        if (leaf) (void)leaf_test<false, COUNT>(sc, r, lref, f, tmin, t.h.t, t.h, cnt);
+        if (leaf) {
+            (void)leaf_test<false, COUNT>(sc, r, lref, f, tmin, t.h.t, t.h, cnt);
+            if (MIXED && any && t.h.leaf >= 0) more = false;
+        }
         busy = more;
     } while (__popcll(__ballot(busy)) > (unsigned)keep);
 }

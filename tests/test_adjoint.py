@@ -234,3 +234,35 @@ def test_gpu_adjoint_beyond_the_lds_accumulators():
     for mine, ref in ((gR[:256], oR[:256]), (gR[256:], oR[256:]), (gL, oL)):
         assert np.linalg.norm(ref) > 0
         assert np.linalg.norm(mine - ref) <= 2e-2 * np.linalg.norm(ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("renderer", ["pt", "ptdirect"])
+@pytest.mark.parametrize("tiles,lights", [(1, 1), (3, 255), (300, 1), (20, 257), (300, 300)])
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (5, 13, 1), (40, 40, 32)])
+def test_gpu_adjoint_slots_and_launch_sizes(renderer, tiles, lights, w, h, spp):
+    """Fewer and more primitives and lights than a block has accumulators,
+    single paths and many, a black tile: the resumable kernel (wide BVH) and
+    the one in which every lane finishes its own paths (binary BVH) agree."""
+    from tests import scenes
+    B = scenes.SceneBuilder()
+    rng = np.random.default_rng(tiles + lights)
+    for i in range(tiles):
+        R = (0.0, 0.5, 0.0) if i == 0 and tiles == 20 else tuple(rng.uniform(0.2, 0.9, 3))
+        B.rect(B.prim(type=ngi.PRIM_D, D_R=R), (-1 + (2 * i + 1) / tiles, 0, 0), (0, 1, 0), (1, 0, 0), 1 / tiles, 1)
+    for i in range(lights):
+        pid = B.prim(type=ngi.PRIM_L | ngi.PRIM_D, light_type=ngi.LIGHT_AREA, Le=tuple(rng.uniform(1, 6, 3)), D_R=(0.5, 0.4, 0.3))
+        B.rect(pid, (-1 + (2 * i + 1) / lights, 1.5, 0), (0, -1, 0), (1, 0, 0), 1 / lights, 0.7)
+    B.camera((0, 1.2, 0.01), (0, 0, 0), up=(0, 0, -1), fov=90.0)
+    s = B.scene(w / h)
+    g = rng.uniform(0.5, 1.5, size=(h, w, 3))
+    out = []
+    for width in (ngi.BVH_2, ngi.BVH_8):
+        s.build(width)
+        p = _params(renderer, w, h, spp, 6, 3)
+        p.engine = ngi.ENGINE_PERSISTENT
+        gR, gL, _ = ngi.render_adjoint(s, p, g)
+        out.append(np.concatenate([gR.ravel(), gL.ravel()]))
+    # The same paths up to FP32 instruction selection, as the binary and the
+    # wide BVH above.
+    assert np.linalg.norm(out[1] - out[0]) <= 1e-3 * np.linalg.norm(out[0])
