@@ -281,6 +281,9 @@ __device__ __forceinline__ float exp2_bits(uint32_t biased) { return __uint_as_f
 // bit for bit.  Every child's sign bit of far - near is shifted into a miss
 // mask, slot 7 first: a subtraction and a shift instead of a compare, a
 // select and a share of the ors (208 -> 201 VALU instructions per visit).
+// The far plane is scaled by a multiply-add of +0, which makes a far plane of
+// -0 a +0: a ray that starts on a corner of the box (far -0 along one axis,
+// near +0 along another) enters it, as 0 <= 0 says, although -0 - 0 is -0.
 // The mask is inverted and limited to the valid slots once, and permuted to
 // processing order at the end.  Which of two coincident surfaces is hit hangs
 // on the rounding of near against tmax, so near and tmax stay as they are.
@@ -312,7 +315,7 @@ __device__ __forceinline__ uint32_t visit8(const Fetch& f, const RayPre& r, floa
         const float tny = fmaf((float)((wny >> sh) & 0xffu), ay, by), tfy = fmaf((float)((wey >> sh) & 0xffu), ay, by);
         const float tnz = fmaf((float)((wnz >> sh) & 0xffu), az, bz), tfz = fmaf((float)((wez >> sh) & 0xffu), az, bz);
         const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, tmin));
-        const float tf = fminf(fminf(fminf(tfx, tfy), tfz) * NGI_SLAB_SCALE, tmax);
+        const float tf = fminf(fmaf(fminf(fminf(tfx, tfy), tfz), NGI_SLAB_SCALE, 0.0f), tmax);
         miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(tf - tn), 31);
     }
     uint32_t hits = ~miss & (meta >> 24);   // valid slots

@@ -194,6 +194,26 @@ def test_trace_leaf_sizes(width, tris, leaf):
     assert np.array_equal(occluded, g["tri"] != ngi.MISS)
 
 
+@pytest.mark.parametrize("width", [ngi.BVH_2, ngi.BVH_8])
+def test_rays_that_start_on_a_box_corner(width):
+    """Rays from a triangle's vertex at the corner of its box, in every octant
+    and with tmin below 0, hit it at distance 0: the box is entered at +0 along
+    one axis and left at -0 along another."""
+    corner = np.array([0.25, -1.5, 2.0])
+    B = SceneBuilder()
+    p = B.prim(type=ngi.PRIM_D, D_R=(0.5, 0.5, 0.5))
+    B.tri(p, corner, corner + (1.0, 0.25, 0.375), corner + (0.25, 1.0, 0.5))
+    B.camera((0.5, 0.5, 5.0), (0.5, 0.5, 0.0))
+    s = B.scene()
+    s.build(width)
+    octants = np.array([[1 if k & 1 else -1, 1 if k & 2 else -1, 1 if k & 4 else -1] for k in range(8)])
+    d = np.concatenate([octants * w for w in ((0.5, 0.75, 0.25), (1.0, 0.0625, 2.0), (0.125, 3.0, 0.5))])
+    rays = ngi.make_rays(np.broadcast_to(corner, d.shape), d, tmin=-0.5)
+    h = s.trace(rays)
+    assert (h["tri"] == 0).all() and (h["t"] == 0.0).all()
+    assert (s.trace(rays, any_hit=True)["tri"] != ngi.MISS).all()
+
+
 @pytest.mark.parametrize("extra", [0, 1, 70001])
 @pytest.mark.parametrize("kind,detail", [(ngi.GEN_CORNELL, 0), (ngi.GEN_BATCH_ROOM, 3000)])
 def test_trace_many_rays_same_as_few(kind, detail, extra):
