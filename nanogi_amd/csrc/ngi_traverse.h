@@ -13,6 +13,7 @@
 #pragma once
 
 #include "ngi_dev.h"
+#include "ngi_quot.h"
 
 namespace ngi {
 
@@ -48,20 +49,8 @@ __device__ __forceinline__ float guard_dir(float d) {
 
 __device__ __forceinline__ float pick(float a, float b, float c, int k) { return k == 0 ? a : (k == 1 ? b : c); }
 
-// 1.0f / d, bit for bit, for 2^-126 <= |d| < 2^126: one Newton step in
-// fused multiply-adds makes the hardware's 1-ulp reciprocal the correctly
-// rounded one (compared with the IEEE division for every significand at 30
-// exponents and signs).  Three instructions instead of the division's ten.
-__device__ __forceinline__ float rcp_ieee(float d) {
-    const float r = __builtin_amdgcn_rcpf(d);
-    return fmaf(fmaf(-d, r, 1.0f), r, r);
-}
-// n / d, bit for bit, given rd = 1 / d correctly rounded (Markstein), while
-// no step leaves the normal range: 2^-100 <= |n| <= |d| < 2^126.
-__device__ __forceinline__ float div_ieee(float n, float d, float rd) {
-    const float q = n * rd;
-    return fmaf(fmaf(-d, q, n), rd, q);
-}
+// 1.0f / d, bit for bit, in quot_exact's range (ngi_quot.h).
+__device__ __forceinline__ float rcp_ieee(float d) { return rcp_newton(d, __builtin_amdgcn_rcpf(d)); }
 
 __device__ __forceinline__ RayPre make_pre(const TraceRay& r) {
     RayPre p;
@@ -90,10 +79,9 @@ __device__ __forceinline__ RayPre make_pre(const TraceRay& r) {
     p.iy = rcp_ieee(guard_dir(r.dy));
     p.iz = rcp_ieee(guard_dir(r.dz));
     p.sz = pick(p.ix, p.iy, p.iz, kz);
-    p.sx = div_ieee(dx, dz, p.sz);
-    p.sy = div_ieee(dy, dz, p.sz);
-    const float ad = fabsf(dz);
-    if (!(fminf(fabsf(dx), fabsf(dy)) >= 7.8886e-31f && ad >= 1e-20f && ad < 8.5e37f)) {   // 2^-100, guard_dir's bound, 2^126
+    p.sx = div_markstein(dx, dz, p.sz);
+    p.sy = div_markstein(dy, dz, p.sz);
+    if (!quot_exact(fminf(fabsf(dx), fabsf(dy)), dz)) {
         p.ix = 1.0f / guard_dir(r.dx);
         p.iy = 1.0f / guard_dir(r.dy);
         p.iz = 1.0f / guard_dir(r.dz);

@@ -194,6 +194,44 @@ def test_trace_leaf_sizes(width, tris, leaf):
     assert np.array_equal(occluded, g["tri"] != ngi.MISS)
 
 
+@pytest.mark.parametrize("exponent", [-60, -3, 0, 20, 25, 26, 60])
+def test_ray_setup_has_the_bits_of_divisions(exponent):
+    """Hits of one triangle against the watertight test in FP32 with IEEE
+    divisions, bit for bit: directions of any and of the greatest significand,
+    with components from equal to far smaller than the longest."""
+    f = np.float32
+    A, Bv, C = (np.array(v, f) for v in ((-300.0, -200.0, 1.0), (400.0, -250.0, 1.25), (-50.0, 500.0, 0.75)))
+    B = SceneBuilder()
+    p = B.prim(type=ngi.PRIM_D, D_R=(0.5, 0.5, 0.5))
+    B.tri(p, A, Bv, C)
+    B.camera((0.5, 0.5, 5.0), (0.5, 0.5, 0.0))
+    s = B.scene()
+    s.build(ngi.BVH_8)
+    rng = np.random.default_rng(exponent + 100)
+    n = 20000
+    d = (rng.uniform(0.5, 1.0, (n, 3)) * 2.0 ** np.stack([-rng.integers(1, 30, n), -rng.integers(1, 30, n), 0 * np.arange(n)], 1)).astype(f)
+    d[::4, 2] = f(1.0) - f(2.0 ** -24)   # the greatest significand
+    d *= rng.choice([-1, 1], (n, 3)).astype(f)
+    d[:, 2] = np.abs(d[:, 2])
+    o = rng.uniform(-1, 1, (n, 3)).astype(f) * f(0.5)
+    d *= f(2.0) ** f(exponent)
+    g = s.trace(ngi.make_rays(o, d, tmin=0.0, tmax=f(1e30)))
+    assert (d[:, 2] > np.abs(d[:, :2]).max(1)).all()   # z is the longest: the shear's axes are x and y
+    sx, sy, sz = d[:, 0] / d[:, 2], d[:, 1] / d[:, 2], f(1.0) / d[:, 2]
+    sheared = []
+    for v in (A, Bv, C):
+        k = v[None] - o
+        sheared.append((k[:, 0] - sx * k[:, 2], k[:, 1] - sy * k[:, 2], sz * k[:, 2]))
+    (Ax, Ay, Az), (Bx, By, Bz), (Cx, Cy, Cz) = sheared
+    U, V, W = Cx * By - Cy * Bx, Ax * Cy - Ay * Cx, Bx * Ay - By * Ax
+    assert ((U < 0) == (V < 0)).all() and ((V < 0) == (W < 0)).all() and (U != 0).all()
+    rd = f(1.0) / (U + V + W)
+    t = (U * Az + V * Bz + W * Cz) * rd
+    assert (g["tri"] == 0).all()
+    for mine, want in ((g["t"], t), (g["u"], V * rd), (g["v"], W * rd)):
+        assert want.dtype == f and np.array_equal(mine.view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("width", [ngi.BVH_2, ngi.BVH_8])
 def test_rays_that_start_on_a_box_corner(width):
     """Rays from a triangle's vertex at the corner of its box, in every octant
