@@ -470,16 +470,17 @@ int ngi_trace(ngi_scene* s, const ngi_ray* rays, size_t n, ngi_hit* hits, int an
     // Up to a slot of the pinned ring the runtime's own copy is faster (20,000
     // rays in a 500-triangle room 96 us, through the ring 106; 100,000: 252,
     // 245; 1.5M: 3,640, 3,034).
-    if (hb <= NGI_TRACE_DIRECT_BYTES) {
-        NGI_HIP_CHECK(hipMemcpyAsync(hits, dh, hb, hipMemcpyDeviceToHost, d.stream));
-        NGI_HIP_CHECK(hipStreamSynchronize(d.stream));
-        return NGI_OK;
+    if (hb > NGI_TRACE_DIRECT_BYTES) {
+        NGI_HIP_CHECK(hipStreamSynchronize(d.stream));   // before the pinned buffer is taken
+        st = read_pinned(d.stream, hits, hb, [&](size_t at, size_t bytes, void* dst) {
+            NGI_HIP_CHECK(hipMemcpyAsync(dst, reinterpret_cast<const char*>(dh) + at, bytes, hipMemcpyDeviceToHost, d.stream));
+            return (int)NGI_OK;
+        });
+        if (st != NGI_NOT_PINNED) return st;
     }
-    NGI_HIP_CHECK(hipStreamSynchronize(d.stream));   // before the pinned buffer is taken
-    return read_pinned(d.stream, hits, hb, [&](size_t at, size_t bytes, void* dst) {
-        NGI_HIP_CHECK(hipMemcpyAsync(dst, reinterpret_cast<const char*>(dh) + at, bytes, hipMemcpyDeviceToHost, d.stream));
-        return (int)NGI_OK;
-    });
+    NGI_HIP_CHECK(hipMemcpyAsync(hits, dh, hb, hipMemcpyDeviceToHost, d.stream));
+    NGI_HIP_CHECK(hipStreamSynchronize(d.stream));
+    return NGI_OK;
 }
 
 int ngi_trace_device(ngi_scene* s, const ngi_ray* d_rays, size_t n, ngi_hit* d_hits, int any_hit) {

@@ -36,7 +36,10 @@ void resident_scenes(int delta);
 // enqueues the production of bytes [at, at + n) into the pinned buffer `dst`
 // (a copy, or a kernel: the buffer is mapped) and returns an NGI status; at is
 // a multiple of 1 MiB.  The caller has waited for the work before.  Returns an
-// NGI status.
+// NGI status, or NGI_NOT_PINNED, with nothing done, where no memory can be
+// pinned (or NGI_PINNED=0 is in the environment): the caller then copies
+// through the runtime.
+#define NGI_NOT_PINNED (-1)
 int read_pinned(hipStream_t st, void* out, size_t bytes, const std::function<int(size_t at, size_t n, void* dst)>& emit);
 
 // Exclusive use of the pinned buffer for a small exchange: its address, or

@@ -1,4 +1,5 @@
 // Kept device workspaces and the pinned read-back (ngi_mem.h).
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -44,6 +45,8 @@ struct Pinned {
     hipEvent_t done[NGI_PIN_SLOTS] = {};
 
     bool ensure() {   // mu held
+        const char* e = getenv("NGI_PINNED");
+        if (e && !strcmp(e, "0")) return false;
         if (p) return true;
         void* q = nullptr;
         if (hipHostMalloc(&q, NGI_PIN_SLOT * NGI_PIN_SLOTS, hipHostMallocDefault) != hipSuccess) {
@@ -165,7 +168,7 @@ int read_pinned(hipStream_t st, void* out, size_t bytes, const std::function<int
     if (bytes == 0) return NGI_OK;
     Pinned& b = pinned();
     std::lock_guard<std::mutex> lock(b.mu);
-    if (!b.ensure()) return fail(NGI_ERR_OOM, "cannot pin %zu bytes of host memory", NGI_PIN_SLOT * NGI_PIN_SLOTS);
+    if (!b.ensure()) return NGI_NOT_PINNED;
     const size_t chunks = (bytes + NGI_PIN_SLOT - 1) / NGI_PIN_SLOT;
     std::atomic<size_t> emitted{0}, taken{0}, copied[NGI_PIN_SLOTS];
     for (auto& c : copied) c.store(0);   // chunks copied out of the slot so far

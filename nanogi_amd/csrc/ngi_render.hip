@@ -376,7 +376,7 @@ __global__ void film_out(const FilmT* __restrict__ film, double scale, double* _
 }
 
 int read_film(hipStream_t st, const void* film, bool film64, size_t n, double scale, double* out) {
-    return read_pinned(st, out, n * 8, [&](size_t at, size_t bytes, void* dst) {
+    const int rc = read_pinned(st, out, n * 8, [&](size_t at, size_t bytes, void* dst) {
         const size_t i0 = at / 8, m = bytes / 8;
         const unsigned grid = (unsigned)((m + 255) / 256);
         double* o = reinterpret_cast<double*>(dst);
@@ -385,16 +385,30 @@ int read_film(hipStream_t st, const void* film, bool film64, size_t n, double sc
         NGI_HIP_CHECK(hipGetLastError());
         return (int)NGI_OK;
     });
+    if (rc != NGI_NOT_PINNED) return rc;
+    if (film64) {
+        NGI_HIP_CHECK(hipMemcpyAsync(out, film, n * 8, hipMemcpyDeviceToHost, st));
+        NGI_HIP_CHECK(hipStreamSynchronize(st));
+        for (size_t i = 0; i < n; ++i) out[i] *= scale;
+    } else {
+        std::vector<float> tmp(n);
+        NGI_HIP_CHECK(hipMemcpyAsync(tmp.data(), film, n * 4, hipMemcpyDeviceToHost, st));
+        NGI_HIP_CHECK(hipStreamSynchronize(st));
+        for (size_t i = 0; i < n; ++i) out[i] = (double)tmp[i] * scale;
+    }
+    return NGI_OK;
 }
 
 // Variance of the mean of k batch films from their first and second moments.
-__global__ void variance_out(const double* __restrict__ m1, const double* __restrict__ m2, double k, double* __restrict__ out, size_t n) {
+__host__ __device__ __forceinline__ double variance_of(double m1, double m2, double k) {
 #pragma clang fp contract(off)
+    const double mean = m1 / k;
+    const double sv = (m2 - k * mean * mean) / (k - 1.0);   // sample variance of batch means
+    return (sv > 0 ? sv : 0.0) / k;
+}
+__global__ void variance_out(const double* __restrict__ m1, const double* __restrict__ m2, double k, double* __restrict__ out, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double mean = m1[i] / k;
-    const double sv = (m2[i] - k * mean * mean) / (k - 1.0);   // sample variance of batch means
-    out[i] = (sv > 0 ? sv : 0.0) / k;
+    if (i < n) out[i] = variance_of(m1[i], m2[i], k);
 }
 
 template <typename FilmT>
@@ -662,6 +676,14 @@ int Session::get_film(double* out, double* var) {
             NGI_HIP_CHECK(hipGetLastError());
             return (int)NGI_OK;
         });
+        if (st == NGI_NOT_PINNED) {
+            std::vector<double> b(n);
+            NGI_HIP_CHECK(hipMemcpyAsync(var, m1, n * 8, hipMemcpyDeviceToHost, stream()));
+            NGI_HIP_CHECK(hipMemcpyAsync(b.data(), m2, n * 8, hipMemcpyDeviceToHost, stream()));
+            NGI_HIP_CHECK(hipStreamSynchronize(stream()));
+            for (size_t i = 0; i < n; ++i) var[i] = variance_of(var[i], b[i], (double)batches);
+            st = NGI_OK;
+        }
         if (st) return st;
     }
     return NGI_OK;
@@ -675,6 +697,11 @@ int Session::get_stats(ngi_stats* out) {
         NGI_HIP_CHECK(hipMemcpyAsync(dst, counters, bytes, hipMemcpyDeviceToHost, stream()));
         return (int)NGI_OK;
     });
+    if (st == NGI_NOT_PINNED) {
+        NGI_HIP_CHECK(hipMemcpyAsync(c, counters, sizeof(c), hipMemcpyDeviceToHost, stream()));
+        NGI_HIP_CHECK(hipStreamSynchronize(stream()));
+        st = NGI_OK;
+    }
     if (st) return st;
     *out = stats;
     out->samples = (int64_t)c[CNT_SAMPLES];

@@ -96,3 +96,38 @@ def test_threads_render_at_once():
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_results_without_pinned_memory(monkeypatch):
+    """Where no host memory can be pinned (NGI_PINNED=0), films, variances,
+    statistics and hits come back all the same, bit for bit."""
+    s = ngi.Scene.generate(ngi.GEN_CORNELL, 1, 1.0)
+    rays = ngi.make_rays(np.full((70000, 3), 0.5), np.random.default_rng(3).normal(size=(70000, 3)))
+    sessions = []
+    for precision in (ngi.PRECISION_FP32_FP64ACC, ngi.PRECISION_FP32_ALL):
+        se = ngi.Session(s, _params("ptdirect", 300, 200, precision=precision))
+        for _ in range(3):
+            se.render_batch(1)
+        sessions.append(se)
+    b = ngi.Batch([s], [_params("ptdirect", 300, 200)], ngi.batch_opts(block_size=128, blocks_per_cu=2))
+    b.render(0)
+    b.sync()
+
+    def results():
+        out = [b.film(0)]
+        for se in sessions:
+            st = se.stats()
+            out += [*se.film(variance=True), np.array([st["samples"], st["extension_rays"], st["shadow_rays"]])]
+        for n in (50, 70000):   # hits of more than 1 MiB among them
+            out.append(s.trace(rays[:n]).view(np.uint32))
+        return out
+
+    want = results()
+    monkeypatch.setenv("NGI_PINNED", "0")
+    for x, y in zip(want, results()):
+        assert np.abs(x).max() > 0 and np.array_equal(x, y)
+    film, st = ngi.render(s, _params("ptdirect", 300, 200))
+    assert st["samples"] == 60000 and np.abs(film - want[0]).max() <= 1e-9 * np.abs(film).max()
+    b.close()
+    for se in sessions:
+        se.close()
