@@ -276,10 +276,9 @@ int ensure_stage(DeviceScene& d, size_t bytes) {
 // Ray-query kernel: one lane per ray, rays and hits in the public layout.
 // ---------------------------------------------------------------------------
 #define NGI_TRACE_BLOCK 256
-// Host queries of at most this many bytes of rays and hits (1,365 of them)
-// are traced in mapped host memory; hits of at most NGI_TRACE_DIRECT_BYTES are
-// copied back by the runtime, more through the pinned ring.
-#define NGI_TRACE_MAPPED_BYTES 65536u
+// Host queries whose rays and hits fit a pinned block (1,365 of them) are traced
+// in mapped host memory; hits of at most NGI_TRACE_DIRECT_BYTES are copied back
+// by the runtime, more through the pinned ring.
 #define NGI_TRACE_DIRECT_BYTES ((size_t)1 << 20)
 
 template <int WIDTH, bool ANY>
@@ -450,8 +449,8 @@ int ngi_trace(ngi_scene* s, const ngi_ray* rays, size_t n, ngi_hit* hits, int an
     const size_t rb = n * sizeof(ngi_ray), hb = n * sizeof(ngi_hit);
     // A few rays: the kernel reads them from, and writes their hits to, mapped
     // host memory (two transfers less; 64 rays 59 -> 46 us per call).
-    if (rb + hb <= NGI_TRACE_MAPPED_BYTES && d.view.num_tris) {
-        PinnedBuffer buf(rb + hb);
+    if (rb + hb <= NGI_PIN_BLOCK_BYTES && d.view.num_tris) {
+        PinnedBlock buf(rb + hb);
         if (buf.get()) {
             ngi_ray* hr = reinterpret_cast<ngi_ray*>(buf.get());
             ngi_hit* hh = reinterpret_cast<ngi_hit*>(hr + n);
@@ -471,7 +470,7 @@ int ngi_trace(ngi_scene* s, const ngi_ray* rays, size_t n, ngi_hit* hits, int an
     // rays in a 500-triangle room 96 us, through the ring 106; 100,000: 252,
     // 245; 1.5M: 3,640, 3,034).
     if (hb > NGI_TRACE_DIRECT_BYTES) {
-        NGI_HIP_CHECK(hipStreamSynchronize(d.stream));   // before the pinned buffer is taken
+        NGI_HIP_CHECK(hipStreamSynchronize(d.stream));   // before the ring is taken
         st = read_pinned(d.stream, hits, hb, [&](size_t at, size_t bytes, void* dst) {
             NGI_HIP_CHECK(hipMemcpyAsync(dst, reinterpret_cast<const char*>(dh) + at, bytes, hipMemcpyDeviceToHost, d.stream));
             return (int)NGI_OK;

@@ -37,19 +37,22 @@ void resident_scenes(int delta);
 // (a copy, or a kernel: the buffer is mapped) and returns an NGI status; at is
 // a multiple of 1 MiB.  The caller has waited for the work before.  Returns an
 // NGI status, or NGI_NOT_PINNED, with nothing done, where no memory can be
-// pinned (or NGI_PINNED=0 is in the environment): the caller then copies
-// through the runtime.
+// pinned (or NGI_PINNED=0 is in the environment) or another thread reads back:
+// the caller then copies through the runtime, so no thread waits for
+// another's results.
 #define NGI_NOT_PINNED (-1)
 int read_pinned(hipStream_t st, void* out, size_t bytes, const std::function<int(size_t at, size_t n, void* dst)>& emit);
 
-// Exclusive use of the pinned buffer for a small exchange: its address, or
-// null while another thread has it (or for more than it holds).
-class PinnedBuffer {
+// A block of mapped pinned memory for a small exchange, one of 16: its
+// address, or null when all are in use, for more bytes than a block's, or where
+// no memory can be pinned.  The holder may wait for its stream.
+#define NGI_PIN_BLOCK_BYTES ((size_t)65536)
+class PinnedBlock {
 public:
-    explicit PinnedBuffer(size_t bytes);
-    ~PinnedBuffer();
-    PinnedBuffer(const PinnedBuffer&) = delete;
-    PinnedBuffer& operator=(const PinnedBuffer&) = delete;
+    explicit PinnedBlock(size_t bytes);
+    ~PinnedBlock();
+    PinnedBlock(const PinnedBlock&) = delete;
+    PinnedBlock& operator=(const PinnedBlock&) = delete;
     void* get() const { return p; }
 
 private:

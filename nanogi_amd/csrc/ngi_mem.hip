@@ -19,8 +19,15 @@ namespace ngi {
 #define NGI_PIN_SLOT ((size_t)1 << 20)
 #define NGI_PIN_SLOTS 16
 #define NGI_PIN_THREADS 8
+// Blocks of PinnedBlock.
+#define NGI_PIN_BLOCKS 16
 
 namespace {
+
+bool may_pin() {
+    const char* e = getenv("NGI_PINNED");
+    return !(e && !strcmp(e, "0"));
+}
 
 struct Workspaces {
     std::mutex mu;
@@ -45,8 +52,7 @@ struct Pinned {
     hipEvent_t done[NGI_PIN_SLOTS] = {};
 
     bool ensure() {   // mu held
-        const char* e = getenv("NGI_PINNED");
-        if (e && !strcmp(e, "0")) return false;
+        if (!may_pin()) return false;
         if (p) return true;
         void* q = nullptr;
         if (hipHostMalloc(&q, NGI_PIN_SLOT * NGI_PIN_SLOTS, hipHostMallocDefault) != hipSuccess) {
@@ -73,6 +79,12 @@ struct Pinned {
     }
 };
 
+struct Blocks {
+    std::mutex mu;   // never held while the device is waited for
+    char* p = nullptr;
+    uint32_t used = 0;
+};
+
 // Never destroyed: calls may come from other static destructors.
 Workspaces& workspaces() {
     static Workspaces* w = new Workspaces();
@@ -81,6 +93,10 @@ Workspaces& workspaces() {
 Pinned& pinned() {
     static Pinned* p = new Pinned();
     return *p;
+}
+Blocks& blocks() {
+    static Blocks* b = new Blocks();
+    return *b;
 }
 
 }  // namespace
@@ -143,18 +159,38 @@ void resident_scenes(int delta) {
     if (w.scenes > 0) return;
     w.trim();
     Pinned& b = pinned();
-    std::lock_guard<std::mutex> pin(b.mu);
-    b.release();
+    {
+        std::lock_guard<std::mutex> pin(b.mu);
+        b.release();
+    }
+    Blocks& k = blocks();
+    std::lock_guard<std::mutex> small(k.mu);
+    if (k.p && !k.used) {
+        (void)hipHostFree(k.p);
+        k.p = nullptr;
+    }
 }
 
-PinnedBuffer::PinnedBuffer(size_t bytes) {
-    Pinned& b = pinned();
-    if (bytes > NGI_PIN_SLOT * NGI_PIN_SLOTS || !b.mu.try_lock()) return;
-    if (b.ensure()) p = b.p;
-    else b.mu.unlock();
+PinnedBlock::PinnedBlock(size_t bytes) {
+    if (bytes > NGI_PIN_BLOCK_BYTES || !may_pin()) return;
+    Blocks& k = blocks();
+    std::lock_guard<std::mutex> lock(k.mu);
+    if (!k.p && hipHostMalloc(reinterpret_cast<void**>(&k.p), NGI_PIN_BLOCK_BYTES * NGI_PIN_BLOCKS, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        k.p = nullptr;
+        return;
+    }
+    static_assert(NGI_PIN_BLOCKS < 32, "bits of used");
+    const int i = __builtin_ctz(~k.used);
+    if (i >= NGI_PIN_BLOCKS) return;
+    k.used |= 1u << i;
+    p = k.p + NGI_PIN_BLOCK_BYTES * i;
 }
-PinnedBuffer::~PinnedBuffer() {
-    if (p) pinned().mu.unlock();
+PinnedBlock::~PinnedBlock() {
+    if (!p) return;
+    Blocks& k = blocks();
+    std::lock_guard<std::mutex> lock(k.mu);
+    k.used &= ~(1u << ((static_cast<char*>(p) - k.p) / NGI_PIN_BLOCK_BYTES));
 }
 
 // The runtime's copy into pageable memory reads back 7 GB/s, on one thread
@@ -167,8 +203,8 @@ PinnedBuffer::~PinnedBuffer() {
 int read_pinned(hipStream_t st, void* out, size_t bytes, const std::function<int(size_t, size_t, void*)>& emit) {
     if (bytes == 0) return NGI_OK;
     Pinned& b = pinned();
-    std::lock_guard<std::mutex> lock(b.mu);
-    if (!b.ensure()) return NGI_NOT_PINNED;
+    std::unique_lock<std::mutex> lock(b.mu, std::try_to_lock);
+    if (!lock || !b.ensure()) return NGI_NOT_PINNED;
     const size_t chunks = (bytes + NGI_PIN_SLOT - 1) / NGI_PIN_SLOT;
     std::atomic<size_t> emitted{0}, taken{0}, copied[NGI_PIN_SLOTS];
     for (auto& c : copied) c.store(0);   // chunks copied out of the slot so far

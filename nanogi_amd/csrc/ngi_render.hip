@@ -692,17 +692,11 @@ int Session::get_film(double* out, double* var) {
 int Session::get_stats(ngi_stats* out) {
     int st = sync();
     if (st) return st;
-    unsigned long long c[CNT_N];
-    st = read_pinned(stream(), c, sizeof(c), [&](size_t, size_t bytes, void* dst) {
-        NGI_HIP_CHECK(hipMemcpyAsync(dst, counters, bytes, hipMemcpyDeviceToHost, stream()));
-        return (int)NGI_OK;
-    });
-    if (st == NGI_NOT_PINNED) {
-        NGI_HIP_CHECK(hipMemcpyAsync(c, counters, sizeof(c), hipMemcpyDeviceToHost, stream()));
-        NGI_HIP_CHECK(hipStreamSynchronize(stream()));
-        st = NGI_OK;
-    }
-    if (st) return st;
+    unsigned long long here[CNT_N];
+    PinnedBlock block(sizeof(here));
+    const unsigned long long* c = block.get() ? reinterpret_cast<const unsigned long long*>(block.get()) : here;
+    NGI_HIP_CHECK(hipMemcpyAsync(block.get() ? block.get() : here, counters, sizeof(here), hipMemcpyDeviceToHost, stream()));
+    NGI_HIP_CHECK(hipStreamSynchronize(stream()));
     *out = stats;
     out->samples = (int64_t)c[CNT_SAMPLES];
     out->extension_rays = (int64_t)c[CNT_EXT_RAYS];

@@ -3,6 +3,7 @@ size come back whole, one call's leftovers never show in the next, and
 threads may render at once.
 """
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -131,3 +132,55 @@ def test_results_without_pinned_memory(monkeypatch):
     b.close()
     for se in sessions:
         se.close()
+
+
+def test_no_thread_waits_for_anothers_render():
+    """A small query behind a long render on its scene's stream keeps no other
+    thread's statistics and films waiting."""
+    rays = ngi.make_rays(np.full((50, 3), 0.5), np.random.default_rng(3).normal(size=(50, 3)))
+    scenes = [ngi.Scene.generate(ngi.GEN_CORNELL, 1, 1.0) for _ in range(5)]
+    sessions = [ngi.Session(s, _params("pt", 64, 64)) for s in scenes[1:]]
+    for s, se in zip(scenes[1:], sessions):
+        s.trace(rays)
+        se.render(1)
+        se.film()
+    long = _params("ptdirect", 256, 256)
+    long.paths_in_flight = 256   # one block: about a second, and room for the others' kernels
+    ends = {}
+
+    def query():
+        scenes[0].trace(rays)
+        ends["query"] = time.perf_counter()
+
+    def read(i):
+        sessions[i].stats()
+        sessions[i].film()
+        scenes[1 + i].trace(rays)
+        ends[i] = time.perf_counter()
+
+    se = ngi.Session(scenes[0], long)
+    se.render(1)
+    se.sync()
+    spp = 4
+    while True:   # as many samples as take half a second
+        t0 = time.perf_counter()
+        se.render(spp)
+        se.sync()
+        if time.perf_counter() - t0 > 0.5:
+            break
+        spp *= 2
+    start = time.perf_counter()
+    se.render(spp)
+    threads = [threading.Thread(target=query)]
+    threads[0].start()
+    time.sleep(0.1)   # the query has been enqueued
+    threads += [threading.Thread(target=read, args=(i,)) for i in range(4)]
+    for t in threads[1:]:
+        t.start()
+    for t in threads:
+        t.join()
+    se.close()
+    # Streams may share a hardware queue with the long render: not all four.
+    assert min(ends[i] for i in range(4)) < start + 0.75 * (ends["query"] - start)
+    for x in sessions:
+        x.close()
