@@ -1,8 +1,9 @@
 // Device workspaces kept between calls, and results read back through pinned
 // memory.
 //
-// Both serve the whole process (every scene lives on the current device 0),
-// are bounded, and are given back when the last resident scene goes.
+// Both serve the whole process (every scene lives on device 0), are bounded,
+// and are given back when the last resident scene goes (pinned memory the first
+// time only: see GiveBack).
 #pragma once
 
 #include <stddef.h>

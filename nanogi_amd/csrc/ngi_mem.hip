@@ -48,29 +48,51 @@ struct Workspaces {
     }
 };
 
+// Pinned memory is given back with the last resident scene, but only once: a
+// program that has to pin it again holds one scene after another, and fresh
+// pages cost it more than the copies they serve (host queries of 1M rays on a
+// new scene each: 4.6 ms with pages pinned anew, 2.8 with kept ones, 3.2
+// through the runtime).
+struct GiveBack {
+    bool given = false, kept = false;
+    void pinned() { kept = given; }   // memory has been pinned
+    bool due() {                      // the last scene is gone
+        given = true;
+        return !kept;
+    }
+};
+
+// hipHostMalloc, and the events of `done`, on the device of every scene: the
+// calling thread's may be another one.
+char* pin(size_t bytes, hipEvent_t* done = nullptr, int events = 0) {
+    int dev = 0;
+    if (hipGetDevice(&dev) == hipSuccess && dev != 0) (void)hipSetDevice(0);
+    void* q = nullptr;
+    bool ok = hipHostMalloc(&q, bytes, hipHostMallocDefault) == hipSuccess;
+    for (int i = 0; i < events && ok; ++i)
+        if (!done[i] && hipEventCreateWithFlags(&done[i], hipEventDisableTiming) != hipSuccess) {
+            done[i] = nullptr;
+            (void)hipHostFree(q);
+            ok = false;
+        }
+    if (!ok) (void)hipGetLastError();
+    if (dev != 0) (void)hipSetDevice(dev);
+    return ok ? static_cast<char*>(q) : nullptr;
+}
+
 struct Pinned {
     std::mutex mu;   // held while the buffer is in use
     char* p = nullptr;
+    GiveBack back;
     hipEvent_t done[NGI_PIN_SLOTS] = {};
     std::unique_ptr<CopyHelpers> helpers;
 
     bool ensure() {   // mu held
         if (!may_pin()) return false;
         if (p) return true;
-        void* q = nullptr;
-        if (hipHostMalloc(&q, NGI_PIN_SLOT * NGI_PIN_SLOTS, hipHostMallocDefault) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-        for (hipEvent_t& e : done)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-                (void)hipGetLastError();
-                e = nullptr;
-                (void)hipHostFree(q);
-                return false;
-            }
-        p = static_cast<char*>(q);
-        return true;
+        p = pin(NGI_PIN_SLOT * NGI_PIN_SLOTS, done, NGI_PIN_SLOTS);
+        if (p) back.pinned();
+        return p != nullptr;
     }
     void release() {   // mu held
         helpers.reset();
@@ -87,6 +109,7 @@ struct Blocks {
     std::mutex mu;   // never held while the device is waited for
     char* p = nullptr;
     uint32_t used = 0;
+    GiveBack back;
 };
 
 // Never destroyed: calls may come from other static destructors.
@@ -164,12 +187,12 @@ void resident_scenes(int delta) {
     w.trim();
     Pinned& b = pinned();
     {
-        std::lock_guard<std::mutex> pin(b.mu);
-        b.release();
+        std::lock_guard<std::mutex> ring(b.mu);
+        if (b.p && b.back.due()) b.release();
     }
     Blocks& k = blocks();
     std::lock_guard<std::mutex> small(k.mu);
-    if (k.p && !k.used) {
+    if (k.p && !k.used && k.back.due()) {
         (void)hipHostFree(k.p);
         k.p = nullptr;
     }
@@ -179,10 +202,10 @@ PinnedBlock::PinnedBlock(size_t bytes) {
     if (bytes > NGI_PIN_BLOCK_BYTES || !may_pin()) return;
     Blocks& k = blocks();
     std::lock_guard<std::mutex> lock(k.mu);
-    if (!k.p && hipHostMalloc(reinterpret_cast<void**>(&k.p), NGI_PIN_BLOCK_BYTES * NGI_PIN_BLOCKS, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        k.p = nullptr;
-        return;
+    if (!k.p) {
+        k.p = pin(NGI_PIN_BLOCK_BYTES * NGI_PIN_BLOCKS);
+        if (!k.p) return;
+        k.back.pinned();
     }
     static_assert(NGI_PIN_BLOCKS < 32, "bits of used");
     const int i = __builtin_ctz(~k.used);
