@@ -21,7 +21,7 @@ template <typename T>
 hipError_t device_malloc(T** p, size_t bytes) { return device_malloc(reinterpret_cast<void**>(p), bytes); }
 
 // Workspaces of sessions and adjoints (films, counters, shadow rings, queues,
-// records): workspace_free keeps up to 512 MB of them for the next
+// records): workspace_free keeps the newest of them, up to 512 MB, for the next
 // workspace_alloc.  The caller has waited for every kernel that uses a block
 // before it frees it, so a block may move between scenes and streams.
 // Contents are undefined.

@@ -34,19 +34,29 @@ bool may_pin() {
 struct Workspaces {
     std::mutex mu;
     std::unordered_map<void*, size_t> size;   // of every block handed out or kept
-    std::vector<void*> kept;
+    std::vector<void*> kept;                  // oldest first
     size_t kept_bytes = 0;
     int scenes = 0;
 
-    void trim() {
-        for (void* p : kept) {
-            size.erase(p);
-            (void)hipFree(p);
+    // Takes the oldest kept blocks out until at most `bytes` are kept; the
+    // caller frees them once it has let go of mu, since hipFree may wait for
+    // the device.
+    std::vector<void*> trim(size_t bytes) {
+        std::vector<void*> out;
+        size_t n = 0;
+        for (; kept_bytes > bytes; ++n) {
+            kept_bytes -= size[kept[n]];
+            size.erase(kept[n]);
+            out.push_back(kept[n]);
         }
-        kept.clear();
-        kept_bytes = 0;
+        kept.erase(kept.begin(), kept.begin() + (long)n);
+        return out;
     }
 };
+
+void free_all(const std::vector<void*>& blocks) {
+    for (void* p : blocks) (void)hipFree(p);
+}
 
 // Pinned memory is given back with the last resident scene, but only once: a
 // program that has to pin it again holds one scene after another, and fresh
@@ -133,10 +143,12 @@ hipError_t device_malloc(void** p, size_t bytes) {
     if (e != hipErrorOutOfMemory) return e;
     (void)hipGetLastError();
     Workspaces& w = workspaces();
+    std::vector<void*> all;
     {
         std::lock_guard<std::mutex> lock(w.mu);
-        w.trim();
+        all = w.trim(0);
     }
+    free_all(all);
     return hipMalloc(p, bytes);
 }
 
@@ -167,24 +179,35 @@ hipError_t workspace_alloc(void** p, size_t bytes) {
 void workspace_free(void* p) {
     if (!p) return;
     Workspaces& w = workspaces();
-    std::lock_guard<std::mutex> lock(w.mu);
-    const auto it = w.size.find(p);
-    if (it == w.size.end()) return;
-    if (w.scenes > 0 && w.kept_bytes + it->second <= NGI_KEPT_BYTES) {
-        w.kept.push_back(p);
-        w.kept_bytes += it->second;
-        return;
+    std::vector<void*> old;
+    {
+        std::lock_guard<std::mutex> lock(w.mu);
+        const auto it = w.size.find(p);
+        if (it == w.size.end()) return;
+        // The newest block is the likeliest to be wanted again: older ones make
+        // room for it, unless it is more than may be kept by itself.
+        if (w.scenes > 0 && it->second <= NGI_KEPT_BYTES) {
+            w.kept.push_back(p);
+            w.kept_bytes += it->second;
+            old = w.trim(NGI_KEPT_BYTES);
+        } else {
+            w.size.erase(it);
+            old.push_back(p);
+        }
     }
-    w.size.erase(it);
-    (void)hipFree(p);
+    free_all(old);
 }
 
 void resident_scenes(int delta) {
     Workspaces& w = workspaces();
-    std::lock_guard<std::mutex> lock(w.mu);
-    w.scenes += delta;
-    if (w.scenes > 0) return;
-    w.trim();
+    std::vector<void*> all;
+    {
+        std::lock_guard<std::mutex> lock(w.mu);
+        w.scenes += delta;
+        if (w.scenes > 0) return;
+        all = w.trim(0);
+    }
+    free_all(all);
     Pinned& b = pinned();
     {
         std::lock_guard<std::mutex> ring(b.mu);

@@ -2,6 +2,8 @@
 size come back whole, one call's leftovers never show in the next, and
 threads may render at once.
 """
+import ctypes
+import os
 import threading
 import time
 
@@ -214,3 +216,38 @@ def test_one_scene_after_another_costs_no_fresh_pages():
         if alone < 1.7 * beside:
             return
     assert alone < 1.7 * beside
+
+
+def test_kept_workspaces_follow_the_sessions_in_use():
+    """After a session of another size has filled the kept workspaces, those of
+    the sessions in use replace them: the second one allocates nothing.  What is
+    kept stays within its bound."""
+    scene = ngi.Scene.generate(ngi.GEN_CORNELL, 1, 1.0)
+    hip = ctypes.CDLL("libamdhip64.so.7", mode=os.RTLD_NOLOAD)   # the runtime that the library uses
+
+    def free():
+        left, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(left), ctypes.byref(total)) == 0
+        return left.value
+
+    def session(w, h):
+        se = ngi.Session(scene, _params("pt", w, h))
+        for _ in range(2):
+            se.render_batch(1)
+        se.sync()
+        return se
+
+    session(64, 64).close()   # what the first render allocates once
+    before = free()
+    session(3600, 2400).close()     # four films of 207 MB
+    for _ in range(2):
+        session(1500, 1000).close()   # four of 36 MB
+        session(800, 500).close()     # four of 9.6 MB
+        assert before - free() <= 512 << 20
+    for w, h in ((1500, 1000), (800, 500)):
+        idle = free()
+        se = session(w, h)
+        assert free() == idle
+        se.close()
+    scene.close()
+    assert free() >= before
