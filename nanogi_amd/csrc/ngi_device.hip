@@ -197,6 +197,10 @@ int device_prepare(HostScene& s) {
     const float4* nodes = nullptr;
     if ((st = upload(*d, reinterpret_cast<const float4*>(s.bvh.nodes.data()), s.bvh.nodes.size() / 16, &nodes))) return st;
     v.nodes = nodes;
+    const uint32_t zero = 0;
+    const uint32_t* flag = nullptr;
+    if ((st = upload(*d, &zero, 1, &flag))) return st;
+    d->scattered = const_cast<uint32_t*>(flag);
     // Area-light triangles and CDFs, per light primitive.
     std::vector<float4> ltris;
     std::vector<float> cf;
@@ -281,12 +285,14 @@ int ensure_stage(DeviceScene& d, size_t bytes) {
 // by the runtime, more through the pinned ring.
 #define NGI_TRACE_DIRECT_BYTES ((size_t)1 << 20)
 
+// Leaves the call to trace_refill_kernel where `scattered` (null: no such
+// kernel follows) says so.
 template <int WIDTH, bool ANY>
 __global__ void __launch_bounds__(NGI_TRACE_BLOCK) trace_kernel(DevScene sc, const ngi_ray* __restrict__ rays, size_t n,
-                                                                ngi_hit* __restrict__ hits) {
+                                                                ngi_hit* __restrict__ hits, const uint32_t* __restrict__ scattered) {
     extern __shared__ uint32_t stk[];   // sc.stack_entries x block (wide BVH only)
     const size_t i = (size_t)blockIdx.x * NGI_TRACE_BLOCK + threadIdx.x;
-    if (i >= n) return;
+    if (i >= n || (scattered && *scattered)) return;
     const ngi_ray r = rays[i];
     TraceRay tr{r.o[0], r.o[1], r.o[2], r.d[0], r.d[1], r.d[2], r.tmin, r.tmax};
     TraceHit h;
@@ -304,30 +310,68 @@ __global__ void __launch_bounds__(NGI_TRACE_BLOCK) trace_kernel(DevScene sc, con
     hits[i] = o;
 }
 
-// Many rays over the wide BVH: every wavefront takes `per_wave` consecutive
-// rays, and lanes whose rays have finished take the next ones as soon as
-// NGI_TRACE_REFILL of them are idle, so a wavefront waits for its slowest ray
-// once instead of after every 64 (one ray per lane left 11 of 64 lanes active
-// per VALU instruction on incoherent rays).  Visits, tests and results are
-// those of trace_bvh8; an iteration is as in trav8_run.  Bound by the latency
-// of the traversal's loads and by instruction issue.  Measured, us, one ray
-// per lane -> refills (1.5M / 6M rays; closest hit): sphere field with 1.8M
-// triangles 355 -> 314 / 1,070 -> 728, nave 296 -> 252 / 984 -> 809, a room of
-// 4,000 triangles 215 -> 154 / 705 -> 432, Cornell box 94 -> 92 / 304 -> 303;
-// any hit 1,064 -> 706 on 6M of the field's.  Refills of 8 or 24: the same
-// within 3%.
+// Many scattered rays over the wide BVH (rays_scattered; the others are left to
+// trace_kernel, launched behind it): every wavefront takes `per_wave`
+// consecutive rays, and lanes whose rays have finished take the next ones as
+// soon as NGI_TRACE_REFILL of them are idle, so a wavefront waits for its
+// slowest ray once instead of after every 64 (one ray per lane left 11 of 64
+// lanes active per VALU instruction).  Visits, tests and results are those of
+// trace_bvh8; an iteration is as in trav8_run.  Bound by the latency of the
+// traversal's loads and by instruction issue.  Measured, us, one ray per lane ->
+// refills (1.5M / 6M random rays; closest hit): sphere field with 1.8M triangles
+// 355 -> 314 / 1,070 -> 728, nave 296 -> 252 / 984 -> 809, a room of 4,000
+// triangles 215 -> 154 / 705 -> 432; any hit 1,064 -> 706 on 6M of the field's.
+// Refills of 8 or 24: the same within 3%.
 #define NGI_TRACE_REFILL 16
 // Blocks per CU: 2 / 3 / 4 / 5 / 6 took 1,068 / 888 / 787 / 728 / 740 us for
 // the field's 6M rays and 409 / 337 / 342 / 314 / 325 for 1.5M.
 #define NGI_TRACE_WAVES 5
-// From two rays per lane on; with fewer a wavefront's last rays take as long
-// as all of them do (200,000 rays of the field: 162 us one ray per lane, 164
-// with refills; nave 86 and 103).
-#define NGI_TRACE_RAYS_PER_LANE 2
+// From four rays per lane and 256 triangles on.  With fewer rays a wavefront's
+// last ones take as long as all of them do (660,000 scattered rays, one ray per
+// lane / refills, us: nave 163 / 153, its any hit 132 / 125, field 225 / 228),
+// and the rays of a wavefront hardly part among a few triangles (6M, Cornell
+// box 293 / 290, its any hit 221 / 233; 1.4M, rooms of 40 / 100 / 300 triangles
+// 56 / 59, 61 / 64, 130 / 101).
+#define NGI_TRACE_RAYS_PER_LANE 4
+#define NGI_TRACE_MIN_TRIS 256
+
+// Whether the rays of a large call are scattered: at fewer than a quarter of 64
+// places are a ray and those 1 and 8 places on neighbours (origins within a
+// sixteenth of the scene's extent, directions within 25 degrees).  Rays in
+// order, a camera's or the shadow rays of its hits, finish together and hold
+// the same nodes; refills would mix them with new rays at the root and leave
+// the device to a few long wavefronts at the end.  4.2M camera rays, one ray per
+// lane / refills, us: field 470 / 740, nave 420 / 655, room of 4,000 triangles
+// 163 / 270; refills only when a wavefront is empty, and ranges handed out
+// round robin, in pieces of 256 rays by blocks or as the rays before turned
+// out, kept at 0.5 to 1.0 of the former.  Deciding costs a call 3 us (this, and
+// the blocks of the kernel that is not meant).  All lanes of a wavefront call
+// this, and every wavefront finds the same.
+__device__ __forceinline__ bool rays_scattered(const DevScene& sc, const ngi_ray* __restrict__ rays, size_t n) {
+    // Places that follow no row length of an image (multiples of the golden ratio).
+    const size_t i = (size_t)__umul64hi((uint64_t)__lane_id() * 0x9e3779b97f4a7c15ull, (uint64_t)(n - 8));
+    const ngi_ray a = rays[i];
+    const uint32_t meta = __float_as_uint(sc.nodes[0].w);
+    const float ext = 255.0f * fmaxf(fmaxf(exp2_bits(meta & 0xffu), exp2_bits((meta >> 8) & 0xffu)), exp2_bits((meta >> 16) & 0xffu));
+    bool near = true;
+    for (int k = 1; k <= 8; k += 7) {
+        const ngi_ray b = rays[i + k];
+        const float o = fmaxf(fmaxf(fabsf(a.o[0] - b.o[0]), fabsf(a.o[1] - b.o[1])), fabsf(a.o[2] - b.o[2]));
+        const float ab = a.d[0] * b.d[0] + a.d[1] * b.d[1] + a.d[2] * b.d[2];
+        const float aa = a.d[0] * a.d[0] + a.d[1] * a.d[1] + a.d[2] * a.d[2], bb = b.d[0] * b.d[0] + b.d[1] * b.d[1] + b.d[2] * b.d[2];
+        near = near && o <= ext * 0.0625f && ab > 0.0f && ab * ab > 0.82f * aa * bb;
+    }
+    return __popcll(__ballot(near)) < 16;
+}
+
 template <bool ANY>
 __global__ void __launch_bounds__(NGI_TRACE_BLOCK, NGI_TRACE_WAVES) trace_refill_kernel(DevScene sc, const ngi_ray* __restrict__ rays, size_t n,
-                                                                                        ngi_hit* __restrict__ hits, size_t per_wave) {
+                                                                                        ngi_hit* __restrict__ hits, size_t per_wave,
+                                                                                        uint32_t* __restrict__ scattered) {
     extern __shared__ uint32_t stk[];   // sc.stack_entries x block
+    const bool mine = rays_scattered(sc, rays, n);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *scattered = mine ? 1u : 0u;
+    if (!mine) return;
     uint32_t* lds_stack = stk + threadIdx.x;
     const uint32_t lane = __lane_id();
     const size_t wave = (size_t)blockIdx.x * (NGI_TRACE_BLOCK / 64) + (threadIdx.x >> 6);
@@ -409,19 +453,19 @@ int launch_trace(HostScene& s, const ngi_ray* d_rays, size_t n, ngi_hit* d_hits,
     if (d.view.bvh_width == 8) {
         const size_t lds = (size_t)d.view.stack_entries * NGI_TRACE_BLOCK * 4;
         const size_t lanes = (size_t)d.cus * NGI_TRACE_WAVES * NGI_TRACE_BLOCK;
-        if (n >= lanes * NGI_TRACE_RAYS_PER_LANE) {
+        const bool many = n >= lanes * NGI_TRACE_RAYS_PER_LANE && d.view.num_tris >= NGI_TRACE_MIN_TRIS;
+        if (many) {
             const unsigned blocks = (unsigned)d.cus * NGI_TRACE_WAVES;
             const size_t per = (n + (size_t)blocks * (NGI_TRACE_BLOCK / 64) - 1) / ((size_t)blocks * (NGI_TRACE_BLOCK / 64));
-            if (any_hit) trace_refill_kernel<true><<<blocks, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits, per);
-            else trace_refill_kernel<false><<<blocks, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits, per);
-            NGI_HIP_CHECK(hipGetLastError());
-            return NGI_OK;
+            if (any_hit) trace_refill_kernel<true><<<blocks, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits, per, d.scattered);
+            else trace_refill_kernel<false><<<blocks, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits, per, d.scattered);
         }
-        if (any_hit) trace_kernel<8, true><<<grid, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits);
-        else trace_kernel<8, false><<<grid, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits);
+        const uint32_t* scattered = many ? d.scattered : nullptr;
+        if (any_hit) trace_kernel<8, true><<<grid, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits, scattered);
+        else trace_kernel<8, false><<<grid, NGI_TRACE_BLOCK, lds, d.stream>>>(d.view, d_rays, n, d_hits, scattered);
     } else {
-        if (any_hit) trace_kernel<2, true><<<grid, NGI_TRACE_BLOCK, 0, d.stream>>>(d.view, d_rays, n, d_hits);
-        else trace_kernel<2, false><<<grid, NGI_TRACE_BLOCK, 0, d.stream>>>(d.view, d_rays, n, d_hits);
+        if (any_hit) trace_kernel<2, true><<<grid, NGI_TRACE_BLOCK, 0, d.stream>>>(d.view, d_rays, n, d_hits, nullptr);
+        else trace_kernel<2, false><<<grid, NGI_TRACE_BLOCK, 0, d.stream>>>(d.view, d_rays, n, d_hits, nullptr);
     }
     NGI_HIP_CHECK(hipGetLastError());
     return NGI_OK;

@@ -12,6 +12,10 @@ magnitude there: the FP32 test then rounds the ray to the other side of
 the edge (grazing rays on finely tessellated surfaces), and at most 1e-4 of
 the rays may be such cases.
 """
+import ctypes
+import os
+import time
+
 import numpy as np
 import pytest
 
@@ -270,6 +274,95 @@ def test_trace_many_rays_same_as_few(kind, detail, extra):
             assert np.array_equal(many["tri"] == ngi.MISS, few["tri"] == ngi.MISS)
         else:
             assert np.array_equal(many.view(np.uint32), few.view(np.uint32))
+
+
+class _DeviceRays:
+    """Rays and hits in device memory, for ngi_trace_device."""
+
+    def __init__(self, scene, rays):
+        self.scene, self.n = scene, len(rays)
+        scene.trace(rays[:1])
+        self.hip = ctypes.CDLL("libamdhip64.so.7", mode=os.RTLD_NOLOAD)   # the runtime that the library uses
+        self.rays, self.hits = ctypes.c_void_p(), ctypes.c_void_p()
+        assert self.hip.hipMalloc(ctypes.byref(self.rays), ctypes.c_size_t(32 * self.n)) == 0
+        assert self.hip.hipMalloc(ctypes.byref(self.hits), ctypes.c_size_t(16 * self.n)) == 0
+        rays = np.ascontiguousarray(rays)
+        assert self.hip.hipMemcpy(self.rays, rays.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(32 * self.n), 1) == 0
+        assert self.hip.hipDeviceSynchronize() == 0
+
+    def trace(self, any_hit, parts=1):
+        """One call for every part; seconds until the device is idle."""
+        at = [self.n * k // parts for k in range(parts + 1)]
+        t0 = time.perf_counter()
+        for a, b in zip(at, at[1:]):
+            assert ngi.lib().ngi_trace_device(self.scene.handle, ctypes.c_void_p(self.rays.value + 32 * a), b - a,
+                                              ctypes.c_void_p(self.hits.value + 16 * a), int(any_hit)) == ngi.OK
+        assert self.hip.hipDeviceSynchronize() == 0
+        return time.perf_counter() - t0
+
+    def result(self):
+        out = np.zeros((self.n, 4), np.uint32)
+        assert self.hip.hipMemcpy(out.ctypes.data_as(ctypes.c_void_p), self.hits, ctypes.c_size_t(out.nbytes), 2) == 0
+        return out
+
+    def close(self):
+        assert self.hip.hipFree(self.rays) == 0 and self.hip.hipFree(self.hits) == 0
+
+
+def _camera_rays(scene, w, h):
+    c = [p for p in scene.desc()["primitives"] if p["type"] & ngi.PRIM_E][0]
+    eye, center, up = (np.array(c[k], np.float64) for k in ("E_eye", "E_center", "E_up"))
+    z = (eye - center) / np.linalg.norm(eye - center)
+    x = np.cross(up, z) / np.linalg.norm(np.cross(up, z))
+    t = np.tan(np.radians(float(c["E_fov_deg"])) / 2)
+    py, px = np.mgrid[0:h, 0:w]
+    d = ((2 * px + 1) / w - 1)[..., None] * t * x + ((2 * py + 1) / h - 1)[..., None] * t * np.cross(z, x) - z
+    d = d.reshape(-1, 3)
+    return ngi.make_rays(np.broadcast_to(eye, d.shape), d / np.linalg.norm(d, axis=1, keepdims=True))
+
+
+@pytest.mark.parametrize("order", ["scattered", "ordered", "half", "still"])
+@pytest.mark.parametrize("extra", [0, 70001])
+def test_trace_device_large_calls_same_as_parts(order, extra):
+    """Device calls at the smallest size for 256 CUs whose rays are looked at
+    for their order, and larger: random rays, a camera's, half of each, and one
+    ray over and over give what calls of a quarter of the size give."""
+    s = ngi.Scene.generate(ngi.GEN_BATCH_ROOM, 2, 1.0, 3000)
+    n = 256 * 5 * 256 * 4 + extra
+    rays = _random_rays([0.01] * 3, [0.99, 0.99, 2.0], n, 3)
+    cam = _camera_rays(s, 1280, -(-n // 1280))[:n]
+    if order == "ordered":
+        rays = cam
+    elif order == "half":
+        rays[: n // 2] = cam[: n // 2]
+    elif order == "still":
+        rays[:] = cam[n // 2]
+    rays["tmax"][::5] = 0.3
+    d = _DeviceRays(s, rays)
+    for any_hit in (False, True):
+        d.trace(any_hit)
+        whole = d.result()
+        d.trace(any_hit, parts=4)
+        parts = d.result()
+        if any_hit:
+            assert np.array_equal(whole[:, 3] == ngi.MISS, parts[:, 3] == ngi.MISS)
+        else:
+            assert np.array_equal(whole, parts) and (whole[:, 3] != ngi.MISS).any()
+    d.close()
+
+
+def test_rays_in_order_keep_the_gain_of_their_order():
+    """4.2M camera rays of the nave take 0.6 of the time of the same rays
+    shuffled; with refilled lanes the order gained nothing."""
+    s = ngi.Scene.generate(ngi.GEN_NAVE, 1, 1.0)
+    rays = _camera_rays(s, 2048, 2048)
+    took = []
+    for r in (rays, rays[np.random.default_rng(0).permutation(len(rays))]):
+        d = _DeviceRays(s, r)
+        d.trace(False)
+        took.append(min(d.trace(False) for _ in range(20)))
+        d.close()
+    assert took[0] <= 0.8 * took[1]
 
 
 @pytest.mark.parametrize("scale", [1e-3, 1.0, 1e4])
