@@ -191,6 +191,46 @@ __device__ __forceinline__ bool leaf_test(const DevScene& sc, const RayPre& r, i
     return false;
 }
 
+// leaf_test for the binary BVH, whose lanes fetch leaves apart from nodes: two
+// triangles at a time, so that their loads overlap.  Through fetch_child its
+// kernels with two traversals spill more scalar registers and lose: ptdirect on
+// the nave, 512x512 pixels at 32 spp, ms, fetch_child / this: FP64 persistent
+// 31.2 / 28.1, megakernel 37.4 / 35.6 and FP64 57.8 / 55.0, FP32 persistent 27.6
+// / 25.3; bdpt on the field 3.3 / 2.9.
+// Sensitive to its form: with a returned bool in place of `done` and the hit
+// stored by leaf_tri they are 35.6 -> 40.8 and 28.1 -> 31.7 again.
+template <bool ANY, bool COUNT>
+__device__ __forceinline__ void leaf_test_pairs(const DevScene& sc, const RayPre& r, int32_t ref, float tmin, float& tmax, TraceHit& h,
+                                                TraceCounters& cnt, bool& done) {
+    const uint32_t v = (uint32_t)(~ref);
+    const uint32_t first = v >> 4, count = (v & 15u) + 1u;
+    for (uint32_t k = 0; k < count; k += 2) {
+        const uint32_t l0 = first + k;
+        const bool two = k + 1 < count;
+        const uint32_t l1 = two ? l0 + 1 : l0;
+        const float4 a0 = sc.tris[3 * l0], b0 = sc.tris[3 * l0 + 1], c0 = sc.tris[3 * l0 + 2];
+        const float4 a1 = sc.tris[3 * l1], b1 = sc.tris[3 * l1 + 1], c1 = sc.tris[3 * l1 + 2];
+        if (COUNT) cnt.tris += two ? 2u : 1u;
+        float t, u, w;
+        if (tri_test(r, a0, b0, c0, tmin, tmax, t, u, w)) {
+            tmax = t;
+            h.t = t, h.u = u, h.v = w, h.leaf = (int32_t)l0;
+            if (ANY) {
+                done = true;
+                return;
+            }
+        }
+        if (two && tri_test(r, a1, b1, c1, tmin, tmax, t, u, w)) {
+            tmax = t;
+            h.t = t, h.u = u, h.v = w, h.leaf = (int32_t)l1;
+            if (ANY) {
+                done = true;
+                return;
+            }
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Binary BVH, private stack (depth is bounded by the builder).
 // ---------------------------------------------------------------------------
@@ -205,6 +245,7 @@ __device__ bool trace_bvh2(const DevScene& sc, const TraceRay& ray, TraceHit& h,
     int32_t stack[NGI_BVH2_STACK];
     int sp = 0;
     int32_t node = 0;
+    bool done = false;
     for (;;) {
         if (node >= 0) {
             const float4* n = sc.nodes + 4 * (size_t)node;
@@ -240,7 +281,8 @@ __device__ bool trace_bvh2(const DevScene& sc, const TraceRay& ray, TraceHit& h,
                 node = stack[--sp];
             }
         } else {
-            if (leaf_test<ANY, COUNT>(sc, r, node, fetch_child(sc, node), tmin, tmax, h, cnt) && ANY) return true;
+            leaf_test_pairs<ANY, COUNT>(sc, r, node, tmin, tmax, h, cnt, done);
+            if (ANY && done) return true;
             if (sp == 0) break;
             node = stack[--sp];
         }
