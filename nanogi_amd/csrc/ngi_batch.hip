@@ -747,10 +747,9 @@ int Batch::get_film(int i, double* out) {
     if (i < 0 || i >= n()) return fail(NGI_ERR_INVALID_ARG, "scene index %d out of range", i);
     if (!rendered) return fail(NGI_ERR_INVALID_ARG, "the batch has not been rendered");
     const size_t m = film_off[i + 1] - film_off[i];
-    NGI_HIP_CHECK(hipStreamSynchronize(stream));
     // W*H/N scaling (src/nanogi.cpp:434-437).
     const double scale = args[i].path_count ? (double)args[i].npix / (double)args[i].path_count : 0.0;
-    return read_film(stream, film + film_off[i], true, m, scale, out);
+    return read_film(stream, film + film_off[i], true, m, scale, out, false);
 }
 
 int Batch::get_times(double* scene_ms, ngi_stats* stats) {

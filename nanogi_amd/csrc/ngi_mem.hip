@@ -261,6 +261,12 @@ int read_pinned(hipStream_t st, void* out, size_t bytes, const std::function<int
     Pinned& b = pinned();
     std::unique_lock<std::mutex> lock(b.mu, std::try_to_lock);
     if (!lock || !b.ensure()) return NGI_NOT_PINNED;
+    if (bytes <= NGI_PIN_SLOT) {   // one slot: nothing to overlap
+        const int s = emit(0, bytes, b.p);
+        if (hipStreamSynchronize(st) != hipSuccess) return fail(NGI_ERR_DEVICE, "reading results back failed");
+        if (s == NGI_OK) memcpy(out, b.p, bytes);
+        return s;
+    }
     const size_t chunks = (bytes + NGI_PIN_SLOT - 1) / NGI_PIN_SLOT;
     const auto size = [=](size_t k) { return std::min(NGI_PIN_SLOT, bytes - k * NGI_PIN_SLOT); };
     const auto job = std::make_shared<ChunkJob>(chunks, (size_t)NGI_PIN_SLOTS, [&b, out, size](size_t k) {

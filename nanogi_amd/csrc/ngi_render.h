@@ -118,9 +118,9 @@ inline bool persistent_only(int renderer) { return is_light_tracer(renderer) || 
 // precision, engine, roulette, vertex cap, sensor).
 int check_render_params(const ngi_scene* sc, const ngi_render_params& p);
 
-// n film values (FP64, or FP32), scaled, into host memory; the caller has
-// waited for the work that writes the film.
-int read_film(hipStream_t st, const void* film, bool film64, size_t n, double scale, double* out);
+// n film values (FP64, or FP32), scaled, into host memory.  `waited`: the
+// caller has waited for the work on `st` that writes the film.
+int read_film(hipStream_t st, const void* film, bool film64, size_t n, double scale, double* out, bool waited);
 
 struct Session {
     ngi_scene* scene = nullptr;

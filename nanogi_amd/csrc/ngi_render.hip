@@ -375,8 +375,20 @@ __global__ void film_out(const FilmT* __restrict__ film, double scale, double* _
     if (i < n) out[i] = (double)film[i] * scale;
 }
 
-int read_film(hipStream_t st, const void* film, bool film64, size_t n, double scale, double* out) {
-    const int rc = read_pinned(st, out, n * 8, [&](size_t at, size_t bytes, void* dst) {
+// A film goes through the pinned buffer, or through the runtime's copy to be
+// finished on the host, whichever is faster.  us per call, FP64 films, runtime /
+// pinned: 26x26 pixels 22 / 14, 28x28 11 / 14, 64x64 16 / 18, 100x100 23 / 24,
+// 120x120 30 / 28, 256x256 130 / 102, 600x600 825 / 433.  An FP32 film is half
+// the bytes to the runtime: 256x256 75 / 101, 500x500 299 / 344, 600x600 458 /
+// 398.
+#define NGI_FILM_TINY ((size_t)16 << 10)
+#define NGI_FILM_PINNED_F64 ((size_t)256 << 10)
+#define NGI_FILM_PINNED_F32 ((size_t)4 << 20)
+int read_film(hipStream_t st, const void* film, bool film64, size_t n, double scale, double* out, bool waited) {
+    const size_t raw = n * (film64 ? 8 : 4);
+    const bool pinned = raw < NGI_FILM_TINY || raw >= (film64 ? NGI_FILM_PINNED_F64 : NGI_FILM_PINNED_F32);
+    if (pinned && !waited) NGI_HIP_CHECK(hipStreamSynchronize(st));   // before the pinned buffer is taken
+    const int rc = !pinned ? NGI_NOT_PINNED : read_pinned(st, out, n * 8, [&](size_t at, size_t bytes, void* dst) {
         const size_t i0 = at / 8, m = bytes / 8;
         const unsigned grid = (unsigned)((m + 255) / 256);
         double* o = reinterpret_cast<double*>(dst);
@@ -663,7 +675,7 @@ int Session::get_film(double* out, double* var) {
     const double scale = paths_done ? (double)npix / (double)paths_done : 0.0;
     // Both are finished on the device, in FP64, on their way out.
     if (out) {
-        st = read_film(stream(), film, film64, n, scale, out);
+        st = read_film(stream(), film, film64, n, scale, out, true);
         if (st) return st;
     }
     if (var) {

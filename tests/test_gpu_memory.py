@@ -251,3 +251,17 @@ def test_kept_workspaces_follow_the_sessions_in_use():
         se.close()
     scene.close()
     assert free() >= before
+
+
+@pytest.mark.parametrize("precision", [ngi.PRECISION_FP32_FP64ACC, ngi.PRECISION_FP32_ALL])
+@pytest.mark.parametrize("pixels", [682, 683, 1365, 1366, 10922, 10923, 43690, 43691, 349525, 349526])
+def test_films_are_the_same_by_either_way_back(monkeypatch, pixels, precision):
+    """Films around the sizes at which their way back changes (16 and 256 KiB, 1
+    and 4 MiB of pixels) have the bits of the runtime's copy, scaled."""
+    s = ngi.Scene.generate(ngi.GEN_CORNELL, 1, 1.0)
+    se = ngi.Session(s, _params("pt", pixels, 1, precision=precision))
+    se.render(3)
+    film = se.film()
+    monkeypatch.setenv("NGI_PINNED", "0")
+    assert film.max() > 0 and np.array_equal(film, se.film())
+    se.close()
