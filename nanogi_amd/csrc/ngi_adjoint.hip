@@ -692,7 +692,7 @@ int render_adjoint(ngi_scene* scene, const ngi_render_params& p, const double* d
     }
     grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(grid, (total + NGI_ADJ_BLOCK - 1) / NGI_ADJ_BLOCK));
     a.path_count = total;
-    persistent_feed(a, NGI_ADJ_BLOCK, 0, false, &grid);
+    persistent_feed(a, NGI_ADJ_BLOCK, 0, false, &grid, ~0ull);   // a replayed path lasts longer than a take
     g.lanes = grid * NGI_ADJ_BLOCK;
     void *d_dl = nullptr, *d_rec = nullptr, *d_gR = nullptr, *d_gL = nullptr, *d_next = nullptr;
     void *d_rp = nullptr, *d_rl = nullptr, *d_zm = nullptr;

@@ -51,24 +51,36 @@ inline int persistent_grid(const void* kern, int block, size_t lds, uint64_t pat
 }
 
 // Feed of a persistent launch of `grid` blocks of which the device holds
-// `full` lanes.  A chunk (RenderArgs::path_chunk) is at most a quarter of a
-// wavefront's share of the paths: chunks of 128 gave a launch of one path per
-// lane to half of its wavefronts, twice 64 paths one after the other (58,000
-// paths in a 2k-triangle room: 375 -> 252 us).  A launch that leaves half of
-// the device's lanes unused runs (`spread`, resumable kernels) on twice the
-// wavefronts with 32 paths each, which wait for the slowest of 32 rays instead
-// of 64 (whole ngi_render calls, us: 14,400 paths on the nave 421 -> 357, pt
-// 317 -> 280; 28,800 on a 90k-triangle sphere field 424 -> 399; 58,000 in the
-// room 343 -> 334; with 16 paths each 401, 321, 387, 391: more wavefronts
-// issue more instructions for the same paths).
-inline void persistent_feed(RenderArgs& a, int block, uint64_t full, bool spread, unsigned* grid) {
-    const uint64_t blocks = (2 * a.path_count + block - 1) / block;
-    if (spread && blocks * block <= full) {
+// `full` lanes.
+//
+// A chunk (RenderArgs::path_chunk) is at most a quarter of a wavefront's share of
+// the paths: chunks of 128 gave a launch of one path per lane to half of its
+// wavefronts, twice 64 paths one after the other (50,000 ptdirect paths in a
+// 2k-triangle room: 1.54 times the speed, Cornell box 1.39).  But it is never so
+// small that the launch's counter is asked more than `takes` times: the counter
+// answers one wavefront after another, 3 to 4 ns each, and paths that end after
+// a vertex or two are done sooner (roulette from the first vertex, a room of 30
+// triangles, times the speed of chunks of 128: pt, 150,000 paths, 0.85 with up to
+// 4,096 takes, 0.87 with 2,048, 1.07 with 1,024; ltdirect, 210,000 paths, 0.76,
+// 0.94, 1.01).
+//
+// A launch that needs less than a tenth of the device's lanes runs (`spread`,
+// resumable kernels) on twice the wavefronts with 32 paths each, which wait for
+// the slowest of 32 rays instead of 64.  16,000 paths, times the speed before the
+// chunk rule, 64 / 32 paths per wavefront: ptdirect on the nave 1.16 / 1.33,
+// ltdirect 1.12 / 1.31, ptdirect in the 2k-triangle room 1.50 / 1.76, pt in the
+// room of 30 triangles 1.20 / 1.18; 50,000: nave 1.10 / 1.13, ltdirect on a
+// 28k-triangle sphere field 1.07 / 1.02; 150,000: nave 1.11 / 0.94, field 1.08 /
+// 0.84.  (More wavefronts issue more instructions for the same paths.)
+#define NGI_FEED_TAKES 1024u
+inline void persistent_feed(RenderArgs& a, int block, uint64_t full, bool spread, unsigned* grid, uint64_t takes = NGI_FEED_TAKES) {
+    if (spread && 10 * a.path_count <= full) {
         a.path_lanes = 32;
-        *grid = (unsigned)blocks;
+        *grid = (unsigned)((2 * a.path_count + block - 1) / block);
     }
     const uint64_t waves = (uint64_t)*grid * (block / 64);
-    if (a.path_chunk) a.path_chunk = (uint32_t)std::min<uint64_t>(a.path_chunk, std::max<uint64_t>(1, a.path_count / (4 * waves)));
+    if (a.path_chunk)
+        a.path_chunk = (uint32_t)std::min<uint64_t>(a.path_chunk, std::max<uint64_t>({1, a.path_count / (4 * waves), a.path_count / takes}));
 }
 
 // Device scratch owned by a session and grown on demand (per-lane bdpt
