@@ -147,7 +147,10 @@ __global__ void __launch_bounds__(NGI_MK_BLOCK, CHUNKED && DIRECT ? NGI_PK_WAVES
 // 1,504; glossy keep 6 / 8 / 10 on the sphere field: 1,861 / 1,863 / 1,867.
 // Once the launch has no paths left a quarter of the busy lanes wait: the
 // wavefront's last paths follow one another less (58,000 paths in a 2k-triangle
-// room: 258 us with none left waiting, 252 with a quarter, 267 with half).
+// room: 258 us with none left waiting, 252 with a quarter, 267 with half; pt on
+// the nave gains 4%).  Not in FP64 ptdirect kernels that take chunks: 400,000
+// paths, none / a quarter, us: Cornell box 512 / 533, room of 100 triangles 505 /
+// 522; 16,000 to 4M in rooms of 300 to 4,000 triangles 3%.
 //
 // FP64 shading (R = double) parks its direction and roulette number in FP64
 // and queues its shadow rays with FP64 contributions (four float4s per
@@ -255,8 +258,8 @@ __global__ void __launch_bounds__(NGI_MK_BLOCK, (resume_waves<R, DIRECT, CHUNKED
             // Lanes without a ray load and store back what they parked last.
             Trav8 tv = parked_trav<NGI_MK_BLOCK>(pk);
             const RayPre r = make_pre(extension_ray(ps, parked_dir_r<NGI_MK_BLOCK, R>(pk)));
-            const int keep = __builtin_amdgcn_readfirstlane(
-                feed.done() ? (int)__popcll(__ballot(busy)) / 4 : (a.sc.any_glossy ? NGI_PK_KEEP : NGI_PK_KEEP_DIFFUSE));
+            const int last = std::is_same<R, double>::value && DIRECT && CHUNKED ? 0 : (int)__popcll(__ballot(busy)) / 4;
+            const int keep = __builtin_amdgcn_readfirstlane(feed.done() ? last : (a.sc.any_glossy ? NGI_PK_KEEP : NGI_PK_KEEP_DIFFUSE));
             trav8_run<COUNT>(a.sc, r, NGI_EPS_F, tv, busy, keep, tc, ext_stk, NGI_MK_BLOCK);
             park_trav<NGI_MK_BLOCK>(pk, tv);
         }
