@@ -283,7 +283,7 @@ int ensure_stage(DeviceScene& d, size_t bytes) {
 // Host queries whose rays and hits fit a pinned block (1,365 of them) are traced
 // in mapped host memory; hits of at most NGI_TRACE_DIRECT_BYTES are copied back
 // by the runtime, more through the pinned ring.
-#define NGI_TRACE_DIRECT_BYTES ((size_t)1 << 20)
+#define NGI_TRACE_DIRECT_BYTES ((size_t)3 << 19)
 
 // Leaves the call to trace_refill_kernel where `scattered` (null: no such
 // kernel follows) says so.
@@ -510,10 +510,12 @@ int ngi_trace(ngi_scene* s, const ngi_ray* rays, size_t n, ngi_hit* hits, int an
     ngi_hit* dh = reinterpret_cast<ngi_hit*>(reinterpret_cast<char*>(d.stage) + rb);
     NGI_HIP_CHECK(hipMemcpyAsync(dr, rays, rb, hipMemcpyHostToDevice, d.stream));
     if ((st = launch_trace(*s, dr, n, dh, any_hit))) return st;
-    // Up to a slot of the pinned ring the runtime's own copy is faster (20,000
-    // rays in a 500-triangle room 96 us, through the ring 106; 100,000: 252,
-    // 245; 1.5M: 3,640, 3,034).
-    if (hb > NGI_TRACE_DIRECT_BYTES) {
+    // Small hits come back faster by the runtime's own copy, which is enqueued
+    // behind the kernel (70,000 rays in a 2k-triangle room 214 us, through the ring
+    // 217; 100,000: 259, 257; 200,000: 487, 438; 700,000: 1,527, 1,300).  So it is
+    // enqueued at once, too, where the ring is not to be had (after waiting 2 to
+    // 12% slower).
+    if (hb > NGI_TRACE_DIRECT_BYTES && pinned_free()) {
         NGI_HIP_CHECK(hipStreamSynchronize(d.stream));   // before the ring is taken
         st = read_pinned(d.stream, hits, hb, [&](size_t at, size_t bytes, void* dst) {
             NGI_HIP_CHECK(hipMemcpyAsync(dst, reinterpret_cast<const char*>(dh) + at, bytes, hipMemcpyDeviceToHost, d.stream));

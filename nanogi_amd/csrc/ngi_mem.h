@@ -42,6 +42,7 @@ void resident_scenes(int delta);
 // the caller then copies through the runtime, so no thread waits for
 // another's results.
 #define NGI_NOT_PINNED (-1)
+bool pinned_free();   // whether read_pinned would start now
 int read_pinned(hipStream_t st, void* out, size_t bytes, const std::function<int(size_t at, size_t n, void* dst)>& emit);
 
 // A block of mapped pinned memory for a small exchange, one of 16: its

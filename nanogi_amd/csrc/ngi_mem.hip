@@ -243,6 +243,12 @@ PinnedBlock::~PinnedBlock() {
     k.used &= ~(1u << ((static_cast<char*>(p) - k.p) / NGI_PIN_BLOCK_BYTES));
 }
 
+bool pinned_free() {
+    Pinned& b = pinned();
+    std::unique_lock<std::mutex> lock(b.mu, std::try_to_lock);
+    return lock && b.ensure();
+}
+
 // The runtime's copy into pageable memory reads back 7 GB/s, on one thread
 // that mostly touches the caller's pages for the first time.  Here the device
 // fills the ring's slots (kernels write finished results straight into mapped

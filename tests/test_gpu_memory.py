@@ -265,3 +265,14 @@ def test_films_are_the_same_by_either_way_back(monkeypatch, pixels, precision):
     monkeypatch.setenv("NGI_PINNED", "0")
     assert film.max() > 0 and np.array_equal(film, se.film())
     se.close()
+
+
+@pytest.mark.parametrize("n", [1365, 1366, 98304, 98305, 150000, 600000])
+def test_hits_are_the_same_by_either_way_back(monkeypatch, n):
+    """Hits around the sizes at which their way back changes (rays in mapped
+    memory, 1.5 MiB of hits) and well above them: each way, the same bits."""
+    s = ngi.Scene.generate(ngi.GEN_BATCH_ROOM, 1, 1.0, 500)
+    rays = ngi.make_rays(np.full((n, 3), 0.5), np.random.default_rng(n).normal(size=(n, 3)))
+    hits = s.trace(rays)
+    monkeypatch.setenv("NGI_PINNED", "0")
+    assert (hits["tri"] != ngi.MISS).any() and np.array_equal(hits.view(np.uint32), s.trace(rays).view(np.uint32))
