@@ -97,7 +97,7 @@ struct DeviceScene {
     void* prim_d_mem = nullptr;
     void* light_f_mem = nullptr;
     void* light_d_mem = nullptr;
-    uint32_t* scattered = nullptr;   // device word: whether the ray query in flight goes to the refilling kernel
+    uint32_t* scattered = nullptr;   // device word, written by every large ray query: whether the refilling kernel takes it
     // Scratch used by ngi_trace for host<->device staging.
     void* stage = nullptr;
     size_t stage_bytes = 0;

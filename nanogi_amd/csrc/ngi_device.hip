@@ -15,6 +15,9 @@
 
 namespace ngi {
 
+// Fewest triangles for trace_refill_kernel.
+#define NGI_TRACE_MIN_TRIS 256
+
 static int device_ready() {
     int n = 0;
     if (hipGetDeviceCount(&n) != hipSuccess || n <= 0) return fail(NGI_ERR_DEVICE, "no HIP device available");
@@ -197,10 +200,10 @@ int device_prepare(HostScene& s) {
     const float4* nodes = nullptr;
     if ((st = upload(*d, reinterpret_cast<const float4*>(s.bvh.nodes.data()), s.bvh.nodes.size() / 16, &nodes))) return st;
     v.nodes = nodes;
-    const uint32_t zero = 0;
-    const uint32_t* flag = nullptr;
-    if ((st = upload(*d, &zero, 1, &flag))) return st;
-    d->scattered = const_cast<uint32_t*>(flag);
+    if (nt >= NGI_TRACE_MIN_TRIS) {
+        NGI_HIP_CHECK(device_malloc(&d->scattered, sizeof(uint32_t)));
+        d->allocs.push_back(d->scattered);
+    }
     // Area-light triangles and CDFs, per light primitive.
     std::vector<float4> ltris;
     std::vector<float> cf;
@@ -333,7 +336,6 @@ __global__ void __launch_bounds__(NGI_TRACE_BLOCK) trace_kernel(DevScene sc, con
 // box 293 / 290, its any hit 221 / 233; 1.4M, rooms of 40 / 100 / 300 triangles
 // 56 / 59, 61 / 64, 130 / 101).
 #define NGI_TRACE_RAYS_PER_LANE 4
-#define NGI_TRACE_MIN_TRIS 256
 
 // Whether the rays of a large call are scattered: at fewer than a quarter of 64
 // places are a ray and those 1 and 8 places on neighbours (origins within a
