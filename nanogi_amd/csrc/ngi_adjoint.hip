@@ -112,7 +112,7 @@ struct AdjPath {
     int nrec;
 };
 
-// A contribution C at pixel `pix` from emitter primitive `emitter_prim`.
+// A contribution C at pixel `pix` from light `light`.
 template <bool ZEROS>
 __device__ __forceinline__ void adj_contribute(const AdjArgs& g, const DevPrim<float>* prims, const DevLight<float>* lights, double* sL,
                                                AdjPath& q, int pix, f3 C, int light) {
@@ -377,8 +377,8 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_WAVES) adjoint_kernel(R
 #define NGI_ADJ_KEEP_DIFFUSE 16
 #endif
 // Parked words of ptdirect behind the extension ray's: direction of the
-// vertex's shadow ray, its contribution, pixel and emitter primitive.
-enum { APK_SX = PK_WORDS, APK_SY, APK_SZ, APK_CX, APK_CY, APK_CZ, APK_PIXEL, APK_EMITTER, APK_WORDS };
+// vertex's shadow ray, its contribution, pixel and light.
+enum { APK_SX = PK_WORDS, APK_SY, APK_SZ, APK_CX, APK_CY, APK_CZ, APK_PIXEL, APK_LIGHT, APK_WORDS };
 template <bool DIRECT, bool ZEROS>
 __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_RESUME_WAVES) adjoint_resume_kernel(RenderArgs a, AdjArgs g, unsigned long long* next) {
     // LDS: the FP64 accumulators, then the traversal stacks
@@ -423,7 +423,7 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_RESUME_WAVES) adjoint_r
             if (parked_hit<NGI_ADJ_BLOCK>(pk).leaf < 0) {
                 const f3 C = f3(__uint_as_float(pk[APK_CX * NGI_ADJ_BLOCK]), __uint_as_float(pk[APK_CY * NGI_ADJ_BLOCK]),
                                 __uint_as_float(pk[APK_CZ * NGI_ADJ_BLOCK]));
-                adj_contribute<ZEROS>(g, prims, lights, sL, q, (int)pk[APK_PIXEL * NGI_ADJ_BLOCK], C, (int)pk[APK_EMITTER * NGI_ADJ_BLOCK]);
+                adj_contribute<ZEROS>(g, prims, lights, sL, q, (int)pk[APK_PIXEL * NGI_ADJ_BLOCK], C, (int)pk[APK_LIGHT * NGI_ADJ_BLOCK]);
             }
             shadow = false;
             if (extends) {
@@ -499,9 +499,9 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_RESUME_WAVES) adjoint_r
                 TraceRay sr;
                 int target;
                 const f3 C = nee_contribution<float>(sc, cam, prims, type, prim, s, wi, T, rn, a.w, a.h, pixel, sr, target);
-                const int emitter = nee_light(sc, rn);
+                const int light = nee_light(sc, rn);
                 if (!is_zero(C) && !geometry) {
-                    adj_contribute<ZEROS>(g, prims, lights, sL, q, target, C, emitter);
+                    adj_contribute<ZEROS>(g, prims, lights, sL, q, target, C, light);
                 } else if (!is_zero(C)) {
                     Trav8 tv;
                     trav8_begin(sr.tmax, tv);
@@ -513,7 +513,7 @@ __global__ void __launch_bounds__(NGI_ADJ_BLOCK, NGI_ADJ_RESUME_WAVES) adjoint_r
                     pk[APK_CY * NGI_ADJ_BLOCK] = __float_as_uint(C.y);
                     pk[APK_CZ * NGI_ADJ_BLOCK] = __float_as_uint(C.z);
                     pk[APK_PIXEL * NGI_ADJ_BLOCK] = (uint32_t)target;
-                    pk[APK_EMITTER * NGI_ADJ_BLOCK] = (uint32_t)emitter;
+                    pk[APK_LIGHT * NGI_ADJ_BLOCK] = (uint32_t)light;
                     shadow = busy = true;
                 }
             }

@@ -319,12 +319,13 @@ __global__ void __launch_bounds__(NGI_TRACE_BLOCK) trace_kernel(DevScene sc, con
 // soon as NGI_TRACE_REFILL of them are idle, so a wavefront waits for its
 // slowest ray once instead of after every 64 (one ray per lane left 11 of 64
 // lanes active per VALU instruction).  Visits, tests and results are those of
-// trace_bvh8; an iteration is as in trav8_run.  Bound by the latency of the
-// traversal's loads and by instruction issue.  Measured, us, one ray per lane ->
-// refills (1.5M / 6M random rays; closest hit): sphere field with 1.8M triangles
-// 355 -> 314 / 1,070 -> 728, nave 296 -> 252 / 984 -> 809, a room of 4,000
-// triangles 215 -> 154 / 705 -> 432; any hit 1,064 -> 706 on 6M of the field's.
-// Refills of 8 or 24: the same within 3%.
+// trace_bvh8; an iteration is as in trav8_run, but that the compiler waits for
+// the next reference before the leaf tests, which do not hide it.  Bound by the
+// latency of the traversal's loads and by instruction issue.  Measured, us, one
+// ray per lane -> refills (1.5M / 6M random rays; closest hit): sphere field with
+// 1.8M triangles 355 -> 314 / 1,070 -> 728, nave 296 -> 252 / 984 -> 809, a room
+// of 4,000 triangles 215 -> 154 / 705 -> 432; any hit 1,064 -> 706 on 6M of the
+// field's.  Refills of 8 or 24: the same within 3%.
 #define NGI_TRACE_REFILL 16
 // Blocks per CU: 2 / 3 / 4 / 5 / 6 took 1,068 / 888 / 787 / 728 / 740 us for
 // the field's 6M rays and 409 / 337 / 342 / 314 / 325 for 1.5M.

@@ -224,8 +224,9 @@ __device__ __forceinline__ void shq_drain(const RenderArgs& a, const ShadowQueue
         }
         if (__ballot(busy) == 0) break;
         // One node visit or leaf per lane, as in trav8_run: the next child is
-        // chosen, and its reference loaded, before the leaves are tested
-        // (Scene::Visible, rt.hpp:2251-2261; src/nanogi.cpp:700-706).
+        // chosen before the leaves are tested (Scene::Visible,
+        // rt.hpp:2251-2261; src/nanogi.cpp:700-706).  Here the compiler waits
+        // for its reference, whose load stands under a branch, before the tests.
         const bool leaf = busy && ref < 0;
         const int32_t lref = ref;
         bool more = busy;

@@ -144,7 +144,9 @@ __device__ __forceinline__ bool tri_test(const RayPre& r, float4 a4, float4 b4, 
 // before -> after: ptdirect on the nave 87.6 -> 84.9
 // (67M paths), 16.8M paths on the sphere field 8.77 -> 8.43, 7.4M with FP64
 // shading 5.12 -> 4.95, adjoint replay on the nave 16.7 -> 15.6, bdpt on the
-// Cornell box 10.04 -> 9.77, 1.5M incoherent rays 0.367 -> 0.342.
+// Cornell box 10.04 -> 9.77, 1.5M incoherent rays 0.367 -> 0.342.  (The
+// pointer is made from an integer, so these are flat loads: they count as LDS
+// accesses too, and the iteration's stack accesses wait for them.)
 typedef uint32_t Word4 __attribute__((ext_vector_type(4)));
 struct Fetch {
     Word4 w[6];
