@@ -359,7 +359,8 @@ int ngi_render_adjoint(ngi_scene* scene, const ngi_render_params* p, const doubl
 /* Scene i's paths are the ones ngi_render draws for params[i] (same   */
 /* seed and stream id give the same image).  scene_ms (optional,       */
 /* num_scenes doubles) receives each scene's completion time in ms     */
-/* after the launch started, from the device wall clock.               */
+/* after the launch started, from the device wall clock.  Scenes run   */
+/* side by side, so most of them complete near the end of the launch.  */
 /* ------------------------------------------------------------------ */
 int ngi_render_batch(ngi_scene* const* scenes, const ngi_render_params* params, int num_scenes,
                      double* const* films, double* scene_ms, ngi_stats* stats);
